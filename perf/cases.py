@@ -66,7 +66,7 @@ def _alineado(L, bits):
 
 def draw(rng):
     tipo = rng.choice(['capa', 'capa', 'capa', 'bloque', 'bloque', 'perdida', 'entreno', 'prompt', 'paso'])
-    d = rng.choice([64, 128, 192, 256, 320, 384, 512, 640, 768])
+    d = rng.choice([64, 96, 256, 384, 512, 768])          # the widths of the named sizes, the benchmark and the tests
     V = rng.choice([256, 1000, 8000, 32000, 32768])
     bits = rng.choice([16, 32])
     if tipo == 'capa':
