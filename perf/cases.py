@@ -183,12 +183,13 @@ def prepare(case, seed):
     tipo = case['tipo']
     if tipo == 'capa':
         x, E, h, gy = _entradas_capa(case, seed, case['L'])
-        g, salida = _grabar(_paso_modulo(_capa(case, seed), [E, h], [x], gy, case['bits']))
-        return dict(tipo=tipo, grafo=g, salida=salida, vivos=(x, E, h, gy))
+        capa = _capa(case, seed)               # the graph reads the weights and the inputs in place: the state keeps them
+        g, salida = _grabar(_paso_modulo(capa, [E, h], [x], gy, case['bits']))
+        return dict(tipo=tipo, grafo=g, salida=salida, vivos=(capa, x, E, h, gy))
     if tipo == 'bloque':
         b, h, gy = _bloque(case, seed)
         g, salida = _grabar(_paso_modulo(b, [h], [], gy, case['bits']))
-        return dict(tipo=tipo, grafo=g, salida=salida, vivos=(h, gy))
+        return dict(tipo=tipo, grafo=g, salida=salida, vivos=(b, h, gy))
     if tipo == 'perdida':
         lg, y = _logits(case, seed)
         return dict(tipo=tipo, lg=lg.requires_grad_(), y=y)
