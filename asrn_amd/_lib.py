@@ -57,6 +57,9 @@ SIGNATURES = {
     'asrn_column_sums_workspace': (_I64, [_I64, _I64]),
     'asrn_column_sums': (ctypes.c_int, [_P, _I32, _I64, _I64, _I64, _P, _P, _I64, _P]),
     'asrn_small_gemm': (ctypes.c_int, [_P, _I64, _I32, _P, _I64, _I32, _P, _I64, _I32, _I32, _I32, _P]),
+    'asrn_gemm_workspace': (_I64, [_I64, _I64, _I64, _I32, _I32, _I32, _I32]),
+    'asrn_gemm': (ctypes.c_int, [_P, _I64, _I32, _P, _I64, _I32, _I32, _P, _I64, _I64, _I64, _I64, _P, _I32, _P, _I32,
+                                 _I32, _P, _I64, _P]),
     'asrn_copy_blocks': (ctypes.c_int, [_I32] + [_P] * 7),
     'asrn_gate_fwd': (ctypes.c_int, [_P, _P, _I32] + [_P] * 11 + [_I64] + [_I32] * 5 + [_F32] * 3 + [_P] * 3),
     'asrn_gate_step': (ctypes.c_int, [_P] * 14 + [_I64] + [_I32] * 5 + [_F32] * 3 + [_P] * 3),

@@ -15,7 +15,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, 'csrc')
 LIB = os.path.join(HERE, 'libasrn_hip.so')
 SOURCES = ['errors.hip', 'bucket_sort.hip', 'ngram.hip', 'scan.hip', 'candidates.hip', 'decode.hip',
-           'decode_produce.hip', 'gate.hip', 'context.hip', 'hidden.hip', 'reduce.hip', 'small_gemm.hip', 'blocks.hip',
+           'decode_produce.hip', 'gate.hip', 'context.hip', 'hidden.hip', 'reduce.hip', 'small_gemm.hip', 'gemm.hip', 'blocks.hip',
            'phi.hip', 'sampling.hip', 'block_step.hip', 'cross_entropy.hip', 'conv_window.hip',
            'layernorm.hip']
 ARCH = os.environ.get('ASRN_OFFLOAD_ARCH', 'gfx950')

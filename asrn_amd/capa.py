@@ -191,11 +191,11 @@ class CapaASRNEstable(nn.Module):
                                  dim=-1))
             filas = E16
         else:
-            y = lineal(E, W, F.pad(pal[0].bias, (0, 2 * mc)))
+            y = lineal(E, W, F.pad(pal[0].bias, (0, 2 * mc)), propio=False)
             hp, za, zb = y.split([m, mc, mc], dim=-1)
             g = F.gelu(torch.cat([hp, _ShiftAdd.apply(za, zb, ctx[0].bias)], dim=-1))
             filas = E
-        phi = lineal(g, W2, b2)
+        phi = lineal(g, W2, b2, propio=False)
         return phi, filas, None
 
     def _contexto(self, h, con_h=False, pesos=None):
@@ -263,7 +263,7 @@ class CapaASRNEstable(nn.Module):
         sorted order, windows and ranks of every table."""
         phi, filas, ids = self._phi_filas(E, pesos, ids=True)
         if partes is not None:                                              # the generation step's value cache
-            v = F.linear(_a_autocast(E), self.v.weight)
+            v = lineal(E, self.v.weight)
             partes.update(phi=phi, V=F.pad(v, (0, 0, 0, 1))[:, 1:])         # V[t] = W_v E[t+1], 0 at the end
         _, order, _, rank, win = ops.bucket_sort(phi.detach(), self.n_tablas, self.n_bits, self.chunk, ids=ids)
         return phi, filas, order, win, rank

@@ -1,0 +1,491 @@
+// Dense products on the bf16 matrix cores with fp32 results: C (M, N) = op(A) op(B) (+ C) (+ bias).
+//
+// fp32 operands (F32): CDNA4's fp32 matrix rate is 157 TFLOP/s, its bf16 rate 16 times that. An fp32 value is exactly
+// the sum of three bf16 values (24 significand bits in three parts of 8, each part the previous remainder rounded to
+// nearest), so a product x y is the sum of nine bf16 products, exact in the fp32 accumulator's input. The three
+// smallest (second x third and below, at most 2^-25 of x y) are left out: six bf16 products per fp32 one, an error
+// below fp32's own rounding of each product, and fewer roundings of the running sum (one per 16 terms and product
+// order). Measured against 64 bits over the declared sizes the results are no further off than the library's fp32
+// products. A value that is not finite, or rounds to infinity in bf16, turns its products into NaN here; results that
+// come out not finite are formed again as plain fp32 sums (redo), so infinities and NaN are those of an fp32 product.
+// bf16 operands (TN only, the weight gradients): the products as they are, summed in fp32.
+//
+// The matrix cores drop the low bits of a sum towards minus infinity (measured: 256 terms leave results low by 1.5e-8
+// of their root mean square on average, whatever their sign, against 2.4e-7 of random error), which a later sum over
+// all tokens would gather. So with the tokens as rows (A not transposed) every other block of rows enters negated and
+// leaves negated again, and the errors of neighbouring blocks cancel (a wave stores whole blocks: one uniform branch).
+//
+// A workgroup of 4 waves forms a BM x BN tile, each wave a quarter of it from 32x32x16 MFMA tiles. Operands are loaded
+// into registers one step ahead, split there and stored to LDS in units of 8 consecutive k of one row, the operand an
+// MFMA lane takes; an operand stored with its rows contiguous (TA, TB) is transposed on the way, 8 k-rows per thread,
+// which costs nothing in fp32 and one permute per pair in bf16. Two workgroups share a CU (50-57 KB of LDS, 256
+// registers a wave): one's loads, splits and barriers run under the other's MFMA.
+// Products with few tiles (weight gradients: K is the token axis) are cut along K: partial products in a workspace,
+// summed in order by a second launch. No atomics: the result is a function of the sizes alone.
+// The weight gradient's bias gradient, the column sums of A (TA), is summed from the values a tile loads anyway.
+#include "common.h"
+
+namespace asrn {
+
+typedef __bf16 bfx2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bfx8 __attribute__((ext_vector_type(8)));
+typedef float fx2 __attribute__((ext_vector_type(2)));
+typedef float fx16 __attribute__((ext_vector_type(16)));
+
+constexpr int kGemmThr = 256;
+
+struct Gemm {
+  const void* A; int64_t lda; const void* B; int64_t ldb;
+  float* C; int64_t ldc;
+  int M, N, K;
+  const float* bias;      // (N) or null
+  int accumulate;         // C += instead of C =
+  float* colsum;          // (M) or null: the sums of A's columns over K (TA)
+  float* part;            // splits > 1: the partial products, one row of `pstride` floats per split
+  int64_t pstride;
+  int splits, kper, tm, tn;
+};
+
+// x, y (NEG: -x, -y) as three bf16 pairs, each the remainder's nearest
+template <bool NEG>
+__device__ __forceinline__ void split3(float x, float y, uint32_t (&p)[3]) {
+  if (NEG) {
+    x = -x;
+    y = -y;
+  }
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    const fx2 v = {x, y};
+    p[i] = __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bfx2));
+    if (i < 2) {
+      x -= __uint_as_float(p[i] << 16);
+      y -= __uint_as_float(p[i] & 0xffff0000u);
+    }
+  }
+}
+
+// One operand's share of a K step: R rows (of op(A), or columns of op(B)) by BK. T: stored with the rows contiguous
+// (element (k, r) at k * ld + r), else with k contiguous. A thread holds U units of 8 consecutive k.
+template <int R, bool T, bool F32, int BK>
+struct Operand {
+  static constexpr int CH = BK / 8;                          // units per row
+  static constexpr int U = R * CH / kGemmThr;                // units per thread
+  static constexpr int PL = F32 ? 3 : 1;                     // bf16 planes
+  // LDS unit of row r in chunk c: bank groups of 8 units. K-contiguous loads write units (c, r) with c fastest, CH to a
+  // row: a chunk stride of 8 / CH mod 8 keeps 8 lanes apart. bf16 transposes write rows 4 apart: a spare unit every 8
+  // rows.
+  static constexpr int CS = F32 ? R + 8 / CH : R + R / 8;
+  static constexpr int UNITS = PL * CH * CS;
+  static __device__ __forceinline__ int at(int p, int c, int r) {
+    return (p * CH + c) * CS + (F32 ? r : r + (r >> 3));
+  }
+  float f[F32 ? U : 1][8];          // F32: the units' values
+  uint32_t w[F32 ? 1 : 8][F32 ? 1 : U / 2];   // bf16: 8 k-rows of U adjacent columns
+
+  static __device__ __forceinline__ void where(int tid, int i, int& c, int& r) {
+    if constexpr (T) {
+      constexpr int G = R / U;
+      c = tid / G;
+      r = (tid % G) * U + i;
+    } else {
+      const int u = tid + kGemmThr * i;
+      c = u % CH;
+      r = u / CH;
+    }
+  }
+  // rows past `rows` repeat the last ones (their results are not stored); k past k1 read as 0
+  template <bool FULL>
+  __device__ __forceinline__ void load(const void* X, int64_t ld, int r0, int rows, int k0, int k1, int tid) {
+    int c, r;
+    where(tid, 0, c, r);
+    if constexpr (F32 && !T) {
+      const float* x = static_cast<const float*>(X);
+#pragma unroll
+      for (int i = 0; i < U; ++i) {
+        where(tid, i, c, r);
+        const int row = r0 + r < rows ? r0 + r : rows - 1, k = k0 + 8 * c;
+        const float* p = x + (int64_t)row * ld + k;
+        float4 lo = make_float4(0.f, 0.f, 0.f, 0.f), hi = lo;
+        if (FULL || k < k1) lo = *reinterpret_cast<const float4*>(p);
+        if (FULL || k + 4 < k1) hi = *reinterpret_cast<const float4*>(p + 4);
+        f[i][0] = lo.x; f[i][1] = lo.y; f[i][2] = lo.z; f[i][3] = lo.w;
+        f[i][4] = hi.x; f[i][5] = hi.y; f[i][6] = hi.z; f[i][7] = hi.w;
+      }
+    } else if constexpr (F32) {
+      const float* x = static_cast<const float*>(X);
+      const int col = r0 + r <= rows - U ? r0 + r : rows - U;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const int k = k0 + 8 * c + j;
+        const bool ok = FULL || k < k1;
+        const float* p = x + (int64_t)(ok ? k : k1 - 1) * ld + col;
+        if constexpr (U == 2) {
+          const float2 v = *reinterpret_cast<const float2*>(p);
+          f[0][j] = ok ? v.x : 0.f;
+          f[1][j] = ok ? v.y : 0.f;
+        } else {
+          const float v = *p;
+          f[0][j] = ok ? v : 0.f;
+        }
+      }
+    } else {
+      const uint16_t* x = static_cast<const uint16_t*>(X);
+      const int col = r0 + r <= rows - U ? r0 + r : rows - U;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const int k = k0 + 8 * c + j;
+        const bool ok = FULL || k < k1;
+        const uint16_t* p = x + (int64_t)(ok ? k : k1 - 1) * ld + col;
+        if constexpr (U == 8) {
+          const uint2 v = *reinterpret_cast<const uint2*>(p), x2 = *reinterpret_cast<const uint2*>(p + 4);
+          w[j][0] = ok ? v.x : 0u;
+          w[j][1] = ok ? v.y : 0u;
+          w[j][2] = ok ? x2.x : 0u;
+          w[j][3] = ok ? x2.y : 0u;
+        } else if constexpr (U == 4) {
+          const uint2 v = *reinterpret_cast<const uint2*>(p);
+          w[j][0] = ok ? v.x : 0u;
+          w[j][1] = ok ? v.y : 0u;
+        } else {
+          const uint32_t v = *reinterpret_cast<const uint32_t*>(p);
+          w[j][0] = ok ? v : 0u;
+        }
+      }
+    }
+  }
+  // rows of a block whose products are formed negated (k-contiguous operands: a wave's 64 / CH rows)
+  static constexpr int BLOCK = kWave / CH;
+  template <bool NEG>
+  __device__ __forceinline__ void store(uint4* lds, int tid) const {
+#pragma unroll
+    for (int i = 0; i < U; ++i) {
+      int c, r;
+      where(tid, i, c, r);
+      if constexpr (F32) {
+        uint32_t q[4][3];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) split3<NEG>(f[i][2 * j], f[i][2 * j + 1], q[j]);
+#pragma unroll
+        for (int p = 0; p < 3; ++p) lds[at(p, c, r)] = make_uint4(q[0][p], q[1][p], q[2][p], q[3][p]);
+      } else {
+        const uint32_t sel = i & 1 ? 0x07060302u : 0x05040100u;   // the high or low halves of two words
+        uint32_t q[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) q[j] = __builtin_amdgcn_perm(w[2 * j + 1][i / 2], w[2 * j][i / 2], sel);
+        lds[at(0, c, r)] = make_uint4(q[0], q[1], q[2], q[3]);
+      }
+    }
+  }
+  // adds this step's values to the thread's U column sums (T)
+  __device__ __forceinline__ void column_sums(float (&s)[U]) const {
+#pragma unroll
+    for (int i = 0; i < U; ++i) {
+      float t = 0.f;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        if constexpr (F32) t += f[i][j];
+        else t += __uint_as_float(i & 1 ? w[j][i / 2] & 0xffff0000u : w[j][i / 2] << 16);
+      }
+      s[i] += t;
+    }
+  }
+};
+
+template <bool T, bool F32>
+__device__ __forceinline__ float element(const void* X, int64_t ld, int r, int k) {
+  const int64_t at = T ? (int64_t)k * ld + r : (int64_t)r * ld + k;
+  if constexpr (F32) return static_cast<const float*>(X)[at];
+  else return __uint_as_float((uint32_t)static_cast<const uint16_t*>(X)[at] << 16);
+}
+
+// k per step: 64 for bf16; for fp32 32, or 64 in the smallest tile, whose few steps wait for their loads
+template <int BM, int BN, bool F32>
+constexpr int step_k() { return !F32 || BM + BN == 128 ? 64 : 32; }
+
+template <int BM, int BN, bool TA, bool TB, bool F32>
+__global__ __launch_bounds__(kGemmThr, 2) void k_gemm(Gemm g) {
+  constexpr int BK = step_k<BM, BN, F32>();
+  using OA = Operand<BM, TA, F32, BK>;
+  using OB = Operand<BN, TB, F32, BK>;
+  constexpr int MI = BM / 64, NI = BN / 64, PL = OA::PL;
+  // the waves' blocks alternate down a tile: 4 waves of BLOCK rows, then the next unit's
+  constexpr bool kSigned = F32 && !TA;
+  __shared__ uint4 lds[OA::UNITS + OB::UNITS];
+  uint4* la = lds;
+  uint4* lb = lds + OA::UNITS;
+  // XCD x takes a contiguous range of tiles, n fastest, then m, then the K slabs: tiles that share rows share its L2
+  const int total = g.tm * g.tn * g.splits, per = (total + kXcdCount - 1) / kXcdCount;
+  const int t = (int)(blockIdx.x % kXcdCount) * per + (int)(blockIdx.x / kXcdCount);
+  if (t >= total) return;
+  const int z = t / (g.tm * g.tn), tile = t % (g.tm * g.tn), bm = tile / g.tn, bn = tile % g.tn;
+  const int tid = threadIdx.x, lane = lane_id(), wave = tid >> 6;
+  const int m0 = bm * BM, n0 = bn * BN, ka = z * g.kper, kb = ka + g.kper < g.K ? ka + g.kper : g.K;
+  const int wm = (wave >> 1) * (BM / 2), wn = (wave & 1) * (BN / 2), lr = lane & 31, lc = lane >> 5;
+  const bool sums = TA && g.colsum != nullptr && bn == 0;
+  float cs[OA::U];
+#pragma unroll
+  for (int i = 0; i < OA::U; ++i) cs[i] = 0.f;
+  fx16 acc[MI][NI];
+#pragma unroll
+  for (int i = 0; i < MI; ++i)
+#pragma unroll
+    for (int j = 0; j < NI; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+  OA a;
+  OB b;
+  auto load = [&](int k) {
+    if (k + BK <= kb) {
+      a.template load<true>(g.A, g.lda, m0, g.M, k, kb, tid);
+      b.template load<true>(g.B, g.ldb, n0, g.N, k, kb, tid);
+    } else {
+      a.template load<false>(g.A, g.lda, m0, g.M, k, kb, tid);
+      b.template load<false>(g.B, g.ldb, n0, g.N, k, kb, tid);
+    }
+  };
+  if (ka < kb) load(ka);
+  for (int k = ka; k < kb; k += BK) {
+    __syncthreads();                              // the last step's LDS reads are done
+    if (kSigned && (wave & 1)) a.template store<true>(la, tid);
+    else a.template store<false>(la, tid);
+    b.template store<false>(lb, tid);
+    if (TA && sums) a.column_sums(cs);
+    __syncthreads();
+    if (k + BK < kb) load(k + BK);                // in flight under this step's products
+#pragma unroll
+    for (int kk = 0; kk < BK / 16; ++kk) {
+      bfx8 fa[MI][PL], fb[NI][PL];
+#pragma unroll
+      for (int p = 0; p < PL; ++p) {
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+          fa[i][p] = __builtin_bit_cast(bfx8, la[OA::at(p, 2 * kk + lc, wm + 32 * i + lr)]);
+#pragma unroll
+        for (int j = 0; j < NI; ++j)
+          fb[j][p] = __builtin_bit_cast(bfx8, lb[OB::at(p, 2 * kk + lc, wn + 32 * j + lr)]);
+      }
+#pragma unroll
+      for (int q = PL - 1; q >= 0; --q)           // the products of parts pa + pb = q, smallest first
+#pragma unroll
+        for (int pa = 0; pa <= q; ++pa)
+#pragma unroll
+          for (int i = 0; i < MI; ++i)
+#pragma unroll
+            for (int j = 0; j < NI; ++j)
+              acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[i][pa], fb[j][q - pa], acc[i][j], 0, 0, 0);
+    }
+  }
+  float* out = g.splits > 1 ? g.part + (int64_t)z * g.pstride : g.C;
+  const int64_t ldo = g.splits > 1 ? g.N : g.ldc;
+  const bool last = g.splits == 1;
+  uint64_t bad = 0;                               // results to form again (bit (i NI + j) 16 + e)
+#pragma unroll
+  for (int i = 0; i < MI; ++i)
+#pragma unroll
+    for (int j = 0; j < NI; ++j) {
+      const int n = n0 + wn + 32 * j + lr;
+      const float bias = last && g.bias && n < g.N ? g.bias[n] : 0.f;
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const int m = m0 + wm + 32 * i + 8 * (e >> 2) + 4 * lc + (e & 3);
+        if (m < g.M && n < g.N) {
+          float v = acc[i][j][e];
+          if (kSigned && ((8 * (e >> 2)) / OA::BLOCK & 1)) v = -v;     // BLOCK is 16 or 8: the block's parity
+          if (F32 && !(fabsf(v) < INFINITY)) {
+            bad |= 1ull << ((i * NI + j) * 16 + e);
+          } else {
+            float* o = out + (int64_t)m * ldo + n;
+            if (last) v += bias;
+            if (last && g.accumulate) v += *o;
+            *o = v;
+          }
+        }
+      }
+    }
+  if constexpr (F32) {
+    while (bad) {                                 // plain fp32 sums, one element at a time (infinities and NaN only)
+      const int x = __ffsll((unsigned long long)bad) - 1;
+      bad &= bad - 1;
+      const int e = x & 15, ij = x >> 4, i = ij / NI, j = ij % NI;
+      const int m = m0 + wm + 32 * i + 8 * (e >> 2) + 4 * lc + (e & 3), n = n0 + wn + 32 * j + lr;
+      float v = 0.f;
+      for (int k = ka; k < kb; ++k)
+        v = fmaf(element<TA, F32>(g.A, g.lda, m, k), element<TB, F32>(g.B, g.ldb, n, k), v);
+      float* o = out + (int64_t)m * ldo + n;
+      if (last && g.bias) v += g.bias[n];
+      if (last && g.accumulate) v += *o;
+      *o = v;
+    }
+  }
+  if constexpr (TA) {
+    if (sums) {                                   // uniform: the chunks' sums of a row combine in order
+      float* red = reinterpret_cast<float*>(lds);
+      __syncthreads();
+#pragma unroll
+      for (int i = 0; i < OA::U; ++i) {
+        int c, r;
+        OA::where(tid, i, c, r);
+        red[c * BM + r] = cs[i];
+      }
+      __syncthreads();
+      if (tid < BM && m0 + tid < g.M) {
+        float v = 0.f;
+#pragma unroll
+        for (int c = 0; c < OA::CH; ++c) v += red[c * BM + tid];
+        (last ? g.colsum : out + (int64_t)g.M * g.N)[m0 + tid] = v;
+      }
+    }
+  }
+}
+
+// C (+)= the sum of the partial products in split order (+ bias), and the column sums behind them. A workgroup takes
+// 32 float4 columns by 8 lanes of splits; the lanes combine in order.
+constexpr int kSumCols = 32, kSumLanes = kGemmThr / kSumCols;
+__global__ __launch_bounds__(kGemmThr) void k_gemm_sum(Gemm g) {
+  __shared__ float4 red[kSumLanes][kSumCols];
+  const int cl = threadIdx.x % kSumCols, sl = threadIdx.x / kSumCols;
+  const int64_t c = ((int64_t)blockIdx.x * kSumCols + cl) * 4, mn = (int64_t)g.M * g.N;
+  const bool live = c < g.pstride;
+  float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
+  if (live) {
+    const float* p = g.part + c;
+    for (int z = sl; z < g.splits; z += 8 * kSumLanes) {
+      float4 v[8];
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        const int y = z + q * kSumLanes;
+        v[q] = *reinterpret_cast<const float4*>(p + (int64_t)(y < g.splits ? y : z) * g.pstride);
+      }
+#pragma unroll
+      for (int q = 0; q < 8; ++q)
+        if (z + q * kSumLanes < g.splits) {
+          s.x += v[q].x; s.y += v[q].y; s.z += v[q].z; s.w += v[q].w;
+        }
+    }
+  }
+  red[sl][cl] = s;
+  __syncthreads();
+  if (sl != 0 || !live) return;
+#pragma unroll
+  for (int l = 1; l < kSumLanes; ++l) {
+    const float4 v = red[l][cl];
+    s.x += v.x; s.y += v.y; s.z += v.z; s.w += v.w;
+  }
+  if (c >= mn) {
+    *reinterpret_cast<float4*>(g.colsum + (c - mn)) = s;
+    return;
+  }
+  const int64_t m = c / g.N, n = c - m * g.N;
+  float* o = g.C + m * g.ldc + n;
+  if (g.bias) { s.x += g.bias[n]; s.y += g.bias[n + 1]; s.z += g.bias[n + 2]; s.w += g.bias[n + 3]; }
+  if (g.accumulate) {
+    const float4 v = *reinterpret_cast<const float4*>(o);
+    s.x += v.x; s.y += v.y; s.z += v.z; s.w += v.w;
+  }
+  *reinterpret_cast<float4*>(o) = s;
+}
+
+struct Plan { int bm, bn, splits, kper; };
+
+static Plan plan_of(int64_t M, int64_t N, int64_t K, bool f32, int tile, int splits) {
+  Plan p;
+  if (tile) {
+    p.bm = tile >> 8;
+    p.bn = tile & 255;
+  } else {
+    p.bm = p.bn = 64;
+    const int64_t t128 = ((M + 127) / 128) * ((N + 127) / 128);
+    if (M > 64 && N > 64 && (t128 >= 448 || (M * N >= 768 * 768 && K >= 2048))) p.bm = p.bn = 128;
+    if (!f32 && M % 8 == 0 && M * N >= 2 << 20) p.bm = 256;   // its threads take 8 columns of A
+  }
+  const int bk = !f32 || p.bm + p.bn == 128 ? 64 : 32;
+  const int64_t tiles = ((M + p.bm - 1) / p.bm) * ((N + p.bn - 1) / p.bn);
+  int64_t s = splits;
+  if (s <= 0) {
+    s = 512 / tiles;
+    const int64_t most = K <= 4096 ? K / 64 : K / 256;
+    if (s > most) s = most;
+    if (tiles >= 128 && K <= 1024) s = 1;
+  }
+  if (s < 1) s = 1;
+  const int64_t steps = (K + bk - 1) / bk;
+  if (s > steps) s = steps > 0 ? steps : 1;
+  p.kper = (int)((steps + s - 1) / s) * bk;
+  p.splits = (int)((K + p.kper - 1) / p.kper);
+  return p;
+}
+
+template <int BM, int BN, bool F32>
+static void launch_tile(bool ta, bool tb, const Gemm& g, unsigned grid, hipStream_t st) {
+  if constexpr (!F32) {
+    hipLaunchKernelGGL((k_gemm<BM, BN, true, true, false>), dim3(grid), dim3(kGemmThr), 0, st, g);
+  } else {
+    if (ta && tb) hipLaunchKernelGGL((k_gemm<BM, BN, true, true, true>), dim3(grid), dim3(kGemmThr), 0, st, g);
+    else if (tb) hipLaunchKernelGGL((k_gemm<BM, BN, false, true, true>), dim3(grid), dim3(kGemmThr), 0, st, g);
+    else hipLaunchKernelGGL((k_gemm<BM, BN, false, false, true>), dim3(grid), dim3(kGemmThr), 0, st, g);
+  }
+}
+
+}  // namespace asrn
+
+using namespace asrn;
+
+extern "C" int64_t asrn_gemm_workspace(int64_t M, int64_t N, int64_t K, int32_t bf16, int32_t colsum, int32_t tile,
+                                       int32_t splits) {
+  if (M < 0 || N < 0 || K < 0) return -1;
+  if (M == 0 || N == 0) return 0;
+  const Plan p = plan_of(M, N, K, !bf16, tile, splits);
+  return p.splits > 1 ? (int64_t)p.splits * (M * N + (colsum ? M : 0)) * 4 : 0;
+}
+
+extern "C" int asrn_gemm(const void* A, int64_t lda, int32_t trans_a, const void* B, int64_t ldb, int32_t trans_b,
+                         int32_t bf16, float* C, int64_t ldc, int64_t M, int64_t N, int64_t K, const float* bias,
+                         int32_t accumulate, float* colsum, int32_t tile, int32_t splits, void* workspace,
+                         int64_t workspace_bytes, void* stream) {
+  // op(A) (M, K): trans_a: stored (K, M). op(B) (K, N): trans_b: stored (N, K)
+  const bool ta = trans_a != 0, rows_b = trans_b == 0;     // rows_b: B's n contiguous
+  ASRN_REQUIRE(M >= 0 && N >= 0 && K >= 1 && M < (1 << 30) && N < (1 << 30) && K < (1 << 30),
+               "asrn_gemm: bad sizes M=%lld N=%lld K=%lld", (long long)M, (long long)N, (long long)K);
+  if (M == 0 || N == 0) return 0;
+  ASRN_REQUIRE(!(ta && !rows_b), "asrn_gemm: A^T B^T is not supported");
+  ASRN_REQUIRE(!bf16 || (ta && rows_b), "asrn_gemm: bf16 operands are for A^T B");
+  ASRN_REQUIRE(N % 4 == 0 && (!ta || M % 4 == 0) && ((ta && rows_b) || K % 4 == 0),
+               "asrn_gemm: N, and M (A transposed) or K (an operand with k contiguous), must be multiples of 4");
+  ASRN_REQUIRE(lda % 4 == 0 && ldb % 4 == 0 && ldc % 4 == 0 && lda >= (ta ? M : K) && ldb >= (rows_b ? N : K) &&
+                   ldc >= N, "asrn_gemm: leading dimensions must be multiples of 4 that hold a row (lda=%lld ldb=%lld "
+               "ldc=%lld)", (long long)lda, (long long)ldb, (long long)ldc);
+  const uintptr_t al = bf16 ? 7 : 15;
+  ASRN_REQUIRE(A && B && C && ((uintptr_t)A & al) == 0 && ((uintptr_t)B & al) == 0 && ((uintptr_t)C & 15) == 0 &&
+                   ((uintptr_t)bias & 15) == 0 && ((uintptr_t)colsum & 15) == 0, "asrn_gemm: misaligned operand");
+  ASRN_REQUIRE(colsum == nullptr || ta, "asrn_gemm: column sums are those of A^T's A");
+  ASRN_REQUIRE(tile == 0 || tile == (128 << 8 | 128) || tile == (64 << 8 | 128) || tile == (128 << 8 | 64) ||
+                   tile == (64 << 8 | 64) || (bf16 && M % 8 == 0 && tile == (256 << 8 | 128)), "asrn_gemm: unknown tile %d", tile);
+  const Plan p = plan_of(M, N, K, !bf16, tile, splits);
+  Gemm g = {A, lda, B, ldb, C, ldc, (int)M, (int)N, (int)K, bias, accumulate ? 1 : 0, colsum, (float*)workspace,
+            M * N + (colsum ? M : 0), p.splits, p.kper, (int)((M + p.bm - 1) / p.bm), (int)((N + p.bn - 1) / p.bn)};
+  const int64_t total = (int64_t)g.tm * g.tn * g.splits;
+  ASRN_REQUIRE(total < (1 << 30), "asrn_gemm: too many tiles");
+  if (p.splits > 1)
+    ASRN_REQUIRE(workspace && workspace_bytes >= p.splits * g.pstride * 4 && ((uintptr_t)workspace & 15) == 0,
+                 "asrn_gemm: needs a 16-byte aligned workspace of %lld bytes (got %lld)",
+                 (long long)(p.splits * g.pstride * 4), (long long)workspace_bytes);
+  hipStream_t st = (hipStream_t)stream;
+  const unsigned grid = (unsigned)((total + kXcdCount - 1) / kXcdCount * kXcdCount);
+  if (bf16) {
+    if (p.bm == 256) launch_tile<256, 128, false>(ta, rows_b, g, grid, st);
+    else if (p.bm == 128 && p.bn == 128) launch_tile<128, 128, false>(ta, rows_b, g, grid, st);
+    else if (p.bm == 128) launch_tile<128, 64, false>(ta, rows_b, g, grid, st);
+    else if (p.bn == 128) launch_tile<64, 128, false>(ta, rows_b, g, grid, st);
+    else launch_tile<64, 64, false>(ta, rows_b, g, grid, st);
+  } else {
+    if (p.bm == 128 && p.bn == 128) launch_tile<128, 128, true>(ta, rows_b, g, grid, st);
+    else if (p.bm == 128) launch_tile<128, 64, true>(ta, rows_b, g, grid, st);
+    else if (p.bn == 128) launch_tile<64, 128, true>(ta, rows_b, g, grid, st);
+    else launch_tile<64, 64, true>(ta, rows_b, g, grid, st);
+  }
+  int rc = check_launch("asrn_gemm");
+  if (rc || p.splits == 1) return rc;
+  const int64_t cols = (g.pstride + 4 * kSumCols - 1) / (4 * kSumCols);
+  hipLaunchKernelGGL(k_gemm_sum, dim3((unsigned)cols), dim3(kGemmThr), 0, st, g);
+  return check_launch("asrn_gemm");
+}

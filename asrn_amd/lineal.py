@@ -1,11 +1,13 @@
-"""Dense projections whose weight gradient fits a long token axis on MI355X.
+"""Dense projections on MI355X: the library's own products (asrn_gemm) where they are the faster ones, and a weight
+gradient that fits a long token axis.
 
 For y = x W^T + b over N tokens, the weight gradient dW = dY^T X reduces over all N (32768 at the layer benchmark's
 shape) into a small (out, in) matrix. As one GEMM it has only (out / tile) x (in / tile) output tiles to spread over
-256 CUs: hipBLASLt ran this layer's weight gradients on 4 to 70 workgroups, at a few percent of the matrix peak, and
-they took a third of the step. Here the token axis is cut into S slabs: one batched GEMM forms the S partial products
-(S times the tiles) and they are added in fp32, in slab order. The forward and the input gradient are the usual
-GEMMs. Under autocast the operands are cast as autocast casts F.linear's, and the products run in that dtype.
+256 CUs. asrn_gemm cuts the token axis into slabs whose partial products are added in order, and sums the bias
+gradient (dY's columns) from the values it loads anyway. fp32 products run there on the bf16 matrix cores, each operand
+split into three bf16 parts: fp32's error at more than fp32's matrix rate. Where hipBLASLt is faster (below), it is
+called as before: the weight gradient as one batched product over slabs of tokens.
+Under autocast the operands are cast as autocast casts F.linear's, and the products run in that dtype.
 
 On the GPU, the sums (the slab partials, and the bias gradients' column sums) run in the library's asrn_column_sums
 (fp32 accumulation in a fixed order, no memset-cleared semaphores, safe to capture in a HIP graph). fp64 operands,
@@ -50,6 +52,61 @@ def _slab(t, s):
     return t.view(s, n // s, k)
 
 
+# fp32 products of fewer multiply-adds than this stay on hipBLASLt, measured (us, it / asrn_gemm): 2048 x 64 x 256
+# 5.9 / 9.1, 4611 x 384 x 192 10.7 / 11.3, 5005 x 256 x 512 19.1 / 17.8, 4611 x 384 x 384 17.6 / 16.0, 32768 x 256 x 256
+# 39.1 / 33.1, 12000 x 768 x 3072 411 / 349: below, a launch's few steps wait for their loads
+MIN_PRODUCTO = 400_000_000
+# fp32 weight gradients over fewer tokens stay there too: 64 x 64 over 200 tokens 7.7 / 9.9, 64 x 256 over 2048 19.0 / 9.6
+MIN_FICHAS = 512
+# bf16 weight gradients on asrn_gemm: weights too large for slab copies (768 x 3072 over 16384 tokens 157 / 129,
+# 1536 x 768 124 / 80) and small ones (112 x 128 12.4 / 11.4, 64 x 1024 over 65536 34 / 32, 512 x 256 over 5008
+# 18.7 / 15.1); between them hipBLASLt's batched slabs win (768 x 768 35 / 51, 512 x 512 over 65536 55 / 69)
+MAX_PESO_16 = 1 << 17
+
+
+def _apto(t):
+    """Whether asrn_gemm can read the 2-D matrix t in place."""
+    return (t.dim() == 2 and t.stride(1) == 1 and t.stride(0) % 4 == 0 and t.stride(0) >= t.shape[1]
+            and t.data_ptr() % (4 * t.element_size()) == 0)
+
+
+def gemm(a, ta, b, tb, out=None, sesgo=None, sumar=False, columnas=False):
+    """op(a) op(b) (+ sesgo) in fp32 on asrn_gemm, op the transpose where ta, tb; sumar: added into out. columnas (ta):
+    returns (product, the sums of a's columns)."""
+    M, K = (a.shape[1], a.shape[0]) if ta else a.shape
+    N = b.shape[0] if tb else b.shape[1]
+    bf = int(a.dtype == torch.bfloat16)
+    if out is None:
+        out = torch.empty((M, N), dtype=torch.float32, device=a.device)
+    cols = torch.empty((M,), dtype=torch.float32, device=a.device) if columnas else None
+    wsb = _lib.query('asrn_gemm_workspace', M, N, K, bf, int(columnas), 0, 0)
+    ws = torch.empty((wsb,), dtype=torch.uint8, device=a.device) if wsb > 0 else None
+    _lib.call('asrn_gemm', _lib.ptr(a), a.stride(0), int(ta), _lib.ptr(b), b.stride(0), int(tb), bf, _lib.ptr(out),
+              out.stride(0), M, N, K, _lib.ptr(sesgo), int(sumar), _lib.ptr(cols), 0, 0, _lib.ptr(ws), wsb,
+              _lib.stream_of(a.device))
+    return (out, cols) if columnas else out
+
+
+def gemm_ok(a, b, tb, sesgo=None):
+    """Whether a @ op(b) (+ sesgo) runs on asrn_gemm: fp32 on the GPU, aligned, MIN_PRODUCTO multiply-adds or more."""
+    (M, K), N = a.shape, b.shape[0 if tb else 1]
+    return (a.is_cuda and a.dtype == b.dtype == torch.float32 and b.device == a.device and M * N * K >= MIN_PRODUCTO
+            and max(M, N, K) < 1 << 30 and N >= 64 and N % 4 == 0 and K % 4 == 0 and _apto(a) and _apto(b)
+            and (sesgo is None or (sesgo.dtype == torch.float32 and sesgo.device == a.device and sesgo.is_contiguous()
+                                   and sesgo.data_ptr() % 16 == 0)))
+
+
+def _gradiente_ok(g2, x2, sesgo):
+    """Whether dW = g2^T x2 runs on asrn_gemm (see the constants above)."""
+    if not (g2.is_cuda and g2.dtype == x2.dtype and g2.dtype in (torch.float32, torch.bfloat16) and _apto(g2)
+            and _apto(x2) and g2.shape[1] % 4 == 0 and x2.shape[1] % 4 == 0 and 1 <= g2.shape[0] < 1 << 30):
+        return False
+    n, peso = g2.shape[0], g2.shape[1] * x2.shape[1]
+    if g2.dtype == torch.float32:
+        return sesgo or n >= MIN_FICHAS
+    return peso >= MAX_SLAB_WEIGHT or peso <= MAX_PESO_16 or slabs_for(n, peso) == 1
+
+
 def _acc_dtype(t):
     return torch.float64 if t.dtype == torch.float64 else torch.float32
 
@@ -77,8 +134,13 @@ def sum_rows(t):
     return t.sum(0, dtype=_acc_dtype(t))
 
 
-def weight_grad(g2, x2):
-    """dW = g2^T x2, summed in fp32 (fp64 for fp64 operands): g2 (N, out), x2 (N, in), both with unit last stride."""
+def weight_grad(g2, x2, sesgo=False):
+    """dW = g2^T x2, summed in fp32 (fp64 for fp64 operands): g2 (N, out), x2 (N, in), both with unit last stride.
+    sesgo: (dW, the bias gradient column_sums(g2))."""
+    if _gradiente_ok(g2, x2, sesgo):
+        return gemm(g2, True, x2, False, columnas=sesgo)
+    if sesgo:
+        return weight_grad(g2, x2), column_sums(g2)
     s = slabs_for(g2.shape[0], g2.shape[1] * x2.shape[1])
     if s == 1:
         return g2.t().mm(x2).to(_acc_dtype(g2))
@@ -96,11 +158,15 @@ def column_sums(g2):
 class _Lineal(torch.autograd.Function):
 
     @staticmethod
-    def forward(ctx, x, w, b, dt):
+    def forward(ctx, x, w, b, dt, propio):
         xc, wc = x.to(dt), w.to(dt)
         bc = b.to(dt) if b is not None else None
-        with torch.autocast(device_type=x.device.type, enabled=False):
-            y = F.linear(xc, wc, bc)
+        x2 = _rows(xc) if propio and xc.is_cuda and xc.dtype == torch.float32 else None
+        if x2 is not None and gemm_ok(x2, wc, True, bc):
+            y = gemm(x2, False, wc, True, sesgo=bc).view(*x.shape[:-1], wc.shape[0])
+        else:
+            with torch.autocast(device_type=x.device.type, enabled=False):
+                y = F.linear(xc, wc, bc)
         ctx.save_for_backward(xc, wc)
         ctx.meta = (x.dtype, w.dtype, None if b is None else b.dtype)
         return y
@@ -114,16 +180,24 @@ class _Lineal(torch.autograd.Function):
             g = g.to(wc.dtype)
             g2 = _rows(g)
             if ctx.needs_input_grad[0]:
-                gx = g.matmul(wc).to(xdt)
+                if gemm_ok(g2, wc, False):
+                    gx = gemm(g2, False, wc, False).view(*g.shape[:-1], wc.shape[1]).to(xdt)
+                else:
+                    gx = g.matmul(wc).to(xdt)
+            con_sesgo = bdt is not None and ctx.needs_input_grad[2]
             if ctx.needs_input_grad[1]:
-                gw = weight_grad(g2, _rows(xc)).to(wdt)
-            if bdt is not None and ctx.needs_input_grad[2]:
+                gw = weight_grad(g2, _rows(xc), con_sesgo)
+                if con_sesgo:
+                    gw, gb = gw[0], gw[1].to(bdt)
+                gw = gw.to(wdt)
+            elif con_sesgo:
                 gb = column_sums(g2).to(bdt)
-        return gx, gw, gb, None
+        return gx, gw, gb, None, None
 
 
-def lineal(x, w, b=None):
-    """F.linear(x, w, b) with the slab-split weight gradient; honours autocast like F.linear."""
+def lineal(x, w, b=None, propio=True):
+    """F.linear(x, w, b) with its products on asrn_gemm where that is faster; honours autocast like F.linear.
+    propio=False: the forward stays F.linear's (outputs whose signs are hashed keep its rounding)."""
     dev = x.device.type
     dt = torch.get_autocast_dtype(dev) if torch.is_autocast_enabled(dev) else x.dtype
-    return _Lineal.apply(x, w, b, dt)
+    return _Lineal.apply(x, w, b, dt, propio)

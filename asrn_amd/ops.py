@@ -13,7 +13,7 @@ import torch.nn.functional as F
 
 from . import _lib
 from ._lib import call, ptr, query, stream_of
-from .lineal import column_sums, weight_grad
+from .lineal import column_sums, gemm, gemm_ok, weight_grad
 
 I32 = torch.int32
 
@@ -215,6 +215,14 @@ class ContextProj(torch.autograd.Function):
 # a0 (the hash MLPs' first layers)
 # ---------------------------------------------------------------------------------------------------------------------
 
+def _sumar_producto(out, a, b):
+    """out += a @ b, fp32, in place."""
+    if gemm_ok(a, b, False) and out.data_ptr() % 16 == 0:
+        gemm(a, False, b, False, out=out, sumar=True)
+    else:
+        out.addmm_(a, b)
+
+
 class Producer(torch.autograd.Function):
     """y = E W^T by one bias-free GEMM, W's rows [W_p (m) | W_a (mc) | W_b (mc)]; returns the hash MLPs' hidden units
     g (B, L, m + mc) = [gelu(W_p E_t + b_word) | gelu(W_a E_t + W_b E_{t-1} + b_ctx)] (asrn_hidden_fwd;
@@ -262,7 +270,7 @@ class Producer(torch.autograd.Function):
             else:
                 # the rows' gradient is a fresh buffer of the candidate backward: accumulate the GEMM into it
                 dE = _c(drows, torch.float32) if drows.dtype != torch.float32 or not drows.is_contiguous() else drows
-                dE.view(B * L, d).addmm_(dy2, W)
+                _sumar_producto(dE.view(B * L, d), dy2, W)
         if ctx.needs_input_grad[1]:
             dW = weight_grad(dy2, E.view(B * L, d))
         if ctx.needs_input_grad[2] or ctx.needs_input_grad[3]:
@@ -351,26 +359,29 @@ class HashProducer(torch.autograd.Function):
             else:
                 # the rows' gradient is a fresh buffer of the candidate backward: accumulate the GEMM into it
                 dE = _c(drows, torch.float32) if drows.dtype != torch.float32 or not drows.is_contiguous() else drows
-                dE.view(B * L, d).addmm_(dy2, W)
+                _sumar_producto(dE.view(B * L, d), dy2, W)
         dW = weight_grad(dy2, E.view(B * L, d)) if ctx.needs_input_grad[1] else None
         return (dE, dW, dbw, dbc, dW2w.view(Pw, m), db2w, dW2c.view(Pc, mc), db2c, None, None, None, None)
 
 
-# products of more multiply-adds than this go to the library GEMM: the one-tile-per-workgroup kernel wins only while
-# the launch, not the arithmetic, is the cost (d = 256: 7 us; d = 768: 70-105 us against about 10 us in the library)
+# products of more multiply-adds than this go to asrn_gemm: the one-tile-per-workgroup kernel wins only while the
+# launch, not the arithmetic, is the cost (d = 256: 7 us; d = 768: 70-105 us)
 SMALL_GEMM_MAX_MACS = 256 ** 3
 
 
-def _mm32(A, B):
-    """fp32 A @ B on the library GEMM, outside any autocast region (operands may be transposed views)."""
+def _mm32(A, B, ta=False, tb=False):
+    """fp32 op(A) @ op(B) (op the transpose where ta, tb) for the products past SMALL_GEMM_MAX_MACS: asrn_gemm, or the
+    library GEMM outside any autocast region where the sizes are not multiples of 4."""
+    if all(x % 4 == 0 for x in (*A.shape, *B.shape)):
+        return gemm(A, ta, B, tb)
     with torch.autocast(device_type=A.device.type, enabled=False):
-        return A.mm(B)
+        return (A.t() if ta else A).mm(B.t() if tb else B)
 
 
 class SmallMatmul(torch.autograd.Function):
     """A @ B for small fp32 matrices (asrn_small_gemm: one workgroup per 16 x 16 tile of the result): the layer's
     W_o W_v. The backward's dA = dC B^T and dB = A^T dC run on the same kernel. Products beyond SMALL_GEMM_MAX_MACS
-    multiply-adds (d > 256) run on the library's fp32 GEMM instead, in both directions."""
+    multiply-adds (d > 256) run on asrn_gemm instead, in both directions."""
 
     @staticmethod
     def forward(ctx, A, B):
@@ -397,9 +408,9 @@ class SmallMatmul(torch.autograd.Function):
         dA = dB = None
         if M * N * K > SMALL_GEMM_MAX_MACS:
             if ctx.needs_input_grad[0]:
-                dA = _mm32(dC, B.t()).to(ctx.dts[0])
+                dA = _mm32(dC, B, tb=True).to(ctx.dts[0])
             if ctx.needs_input_grad[1]:
-                dB = _mm32(A.t(), dC).to(ctx.dts[1])
+                dB = _mm32(A, dC, ta=True).to(ctx.dts[1])
             return dA, dB
         if ctx.needs_input_grad[0]:                # (M, K) = dC (M, N) B^T
             dA = torch.empty((M, K), dtype=torch.float32, device=dev)

@@ -198,6 +198,22 @@ int64_t asrn_column_sums_workspace(int64_t rows, int64_t cols);
 int asrn_column_sums(const void* x, int32_t bf16, int64_t rows, int64_t cols, int64_t ld, float* out,
                      void* workspace, int64_t workspace_bytes, void* stream);
 
+/* ---- dense products ---------------------------------------------------------------------------------------------
+ * No counterpart in the reference's FFI: the products of its nn.Linear projections and their gradients
+ * (asrn/nucleo.py:591-630, 969-1014), which it leaves to the framework's BLAS. C (M, N) fp32 = op(A) op(B) (+ C with
+ * accumulate) (+ bias (N)), row-major with leading dimensions lda, ldb, ldc. bf16 = 0: fp32 operands, A (M, K) or, with
+ * trans_a, stored (K, M); B (K, N) or, with trans_b, stored (N, K); not both. fp32 precision: each operand is split
+ * into three bf16 parts whose products run on the matrix cores. bf16 != 0: bf16 operands, A stored (K, M) and B (K, N),
+ * summed in fp32. colsum (M), with trans_a: also the sums of A's columns over K. N, M (trans_a) and K (an operand with
+ * k contiguous) and the leading dimensions are multiples of 4, fp32 pointers 16-byte and bf16 ones 8-byte aligned.
+ * tile: 0 (chosen by the sizes) or rows << 8 | columns of 64 or 128; splits: 0 (chosen) or the slabs of K summed in
+ * order. workspace: asrn_gemm_workspace bytes (0: none needed). */
+int64_t asrn_gemm_workspace(int64_t M, int64_t N, int64_t K, int32_t bf16, int32_t colsum, int32_t tile,
+                            int32_t splits);
+int asrn_gemm(const void* A, int64_t lda, int32_t trans_a, const void* B, int64_t ldb, int32_t trans_b, int32_t bf16,
+              float* C, int64_t ldc, int64_t M, int64_t N, int64_t K, const float* bias, int32_t accumulate,
+              float* colsum, int32_t tile, int32_t splits, void* workspace, int64_t workspace_bytes, void* stream);
+
 /* ---- products of small matrices ---------------------------------------------------------------------------------
  * No counterpart in the reference's FFI. The layer applies W_o W_v to the gathered sum of embedding rows (the two
  * linear maps the reference applies one after the other, V = v(E shifted) at asrn/nucleo.py:683 and aporte =

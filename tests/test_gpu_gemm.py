@@ -1,0 +1,119 @@
+"""asrn_gemm (the dense products on the bf16 matrix cores, fp32 operands split into three bf16 parts) against float64
+products, and the dispatch in asrn_amd.lineal against F.linear. The error bound: 2^-24 for each operand's product in the
+split, as fp32's own, and the fp32 sum's rounding, which grows as the square root of the number of terms added to the
+accumulator (K / 16 steps of six products): 2^-24 (2 + sqrt(K)) covers both in the 2-norm over random operands."""
+import pytest
+import torch
+
+from asrn_amd import _lib
+from asrn_amd.lineal import gemm, lineal, weight_grad
+
+pytestmark = pytest.mark.gpu
+TILES = [128 << 8 | 128, 64 << 8 | 128, 128 << 8 | 64, 64 << 8 | 64]
+
+
+def _llamar(a, ta, b, tb, M, N, K, out, tile, splits, bias=None, accumulate=0, columns=None):
+    bf = int(a.dtype == torch.bfloat16)
+    n = _lib.query('asrn_gemm_workspace', M, N, K, bf, int(columns is not None), tile, splits)
+    ws = torch.empty(max(n, 16), dtype=torch.uint8, device='cuda')
+    _lib.call('asrn_gemm', _lib.ptr(a), a.stride(0), ta, _lib.ptr(b), b.stride(0), tb, bf, _lib.ptr(out), out.stride(0),
+              M, N, K, _lib.ptr(bias), accumulate, _lib.ptr(columns), tile, splits, _lib.ptr(ws), n,
+              _lib.stream_of(a.device))
+
+
+def _rel(a, b):
+    return ((a.double() - b).norm() / b.norm()).item()
+
+
+@pytest.mark.parametrize('tile', TILES)
+@pytest.mark.parametrize('ta,tb,M,N,K', [(0, 1, 1, 4, 4), (0, 1, 129, 132, 36), (0, 0, 127, 68, 100), (1, 0, 132, 60, 1),
+                                         (1, 0, 4, 128, 333), (0, 0, 300, 260, 516)])
+def test_fp32_matches_float64(tile, ta, tb, M, N, K):
+    g = torch.Generator(device='cuda').manual_seed(M + N + K)
+    r = lambda *s: torch.randn(*s, generator=g, device='cuda')
+    a = r(K, M + 4)[:, 4:] if ta else r(M, K + 8)[:, 4:4 + K]           # offset, wider leading dimensions
+    b = r(N, K + 4)[:, :K] if tb else r(K, N)
+    bias, c0 = r(N), r(M, N + 4)
+    exact = (a.double().t() if ta else a.double()) @ (b.double().t() if tb else b.double())
+    bound = 2.0 ** -24 * (2 + K ** 0.5)
+    for splits in (1, 2, 5):
+        out = torch.full((M, N + 4), 7.0, device='cuda')
+        cols = torch.empty(M, device='cuda') if ta else None
+        _llamar(a, ta, b, tb, M, N, K, out, tile, splits, columns=cols)
+        assert _rel(out[:, :N], exact) <= bound
+        assert bool((out[:, N:] == 7.0).all())
+        if ta:
+            assert _rel(cols, a.double().sum(0)) <= 2.0 ** -24 * (2 + K) * a.abs().sum(0).norm().item() / a.sum(0).norm().item()
+        out.copy_(c0)
+        _llamar(a, ta, b, tb, M, N, K, out, tile, splits, bias=bias, accumulate=1)
+        assert _rel(out[:, :N], exact + bias.double() + c0[:, :N].double()) <= bound + 2.0 ** -22
+
+
+@pytest.mark.parametrize('tile', TILES + [256 << 8 | 128])
+@pytest.mark.parametrize('M,N,K', [(8, 4, 1), (4, 8, 7), (136, 124, 65), (264, 136, 700)])
+def test_bf16_weight_gradient(tile, M, N, K):
+    if tile >> 8 == 256 and M % 8:
+        tile = 0
+    g = torch.Generator(device='cuda').manual_seed(K)
+    a = torch.randn(K, M, generator=g, device='cuda').bfloat16()
+    b = torch.randn(K, N, generator=g, device='cuda').bfloat16()
+    for splits in (1, 3):
+        out, cols = torch.empty(M, N, device='cuda'), torch.empty(M, device='cuda')
+        _llamar(a, 1, b, 0, M, N, K, out, tile, splits, columns=cols)
+        assert _rel(out, a.double().t() @ b.double()) <= 2.0 ** -24 * (2 + K ** 0.5)
+        torch.testing.assert_close(cols.double(), a.double().sum(0), rtol=1e-5, atol=1e-5 * K ** 0.5)
+
+
+def test_infinities_and_nan_are_fp32s():
+    """A row with an infinity, a NaN, and a value that rounds to infinity in bf16, beside finite rows."""
+    g = torch.Generator(device='cuda').manual_seed(0)
+    a, b = torch.randn(130, 64, generator=g, device='cuda'), torch.randn(68, 64, generator=g, device='cuda')
+    a[3, 5], a[7, 9], a[9, 1] = float('inf'), float('nan'), 3.4e38
+    b[:, 1] *= 1e-30
+    ref = a @ b.t()
+    for splits in (1, 2):
+        out = torch.empty(130, 68, device='cuda')
+        _llamar(a, 0, b, 1, 130, 68, 64, out, 0, splits)
+        assert torch.equal(torch.isnan(out), torch.isnan(ref)) and torch.equal(torch.isinf(out), torch.isinf(ref))
+        assert torch.equal(out[3], ref[3])
+        torch.testing.assert_close(out[9], ref[9], rtol=1e-5, atol=0)
+
+
+@pytest.mark.parametrize('N,fin,fout', [(2049, 512, 516), (5003, 768, 128), (700, 64, 64), (700, 63, 65)])
+@pytest.mark.parametrize('dt', [torch.float32, torch.bfloat16])
+def test_lineal_matches_float64(N, fin, fout, dt):
+    """Sizes on both sides of every line of the dispatch, and sizes no own product takes, in a captured graph too."""
+    g = torch.Generator(device='cuda').manual_seed(N)
+    x = torch.randn(N, fin, generator=g, device='cuda').to(dt).requires_grad_()
+    w = (torch.randn(fout, fin, generator=g, device='cuda') / fin ** 0.5).to(dt).requires_grad_()
+    b = torch.randn(fout, generator=g, device='cuda').to(dt).requires_grad_()
+    gy = torch.randn(N, fout, generator=g, device='cuda').to(dt)
+    tol = 2.0 ** -24 * (4 + N ** 0.5) if dt == torch.float32 else 2.0 ** -8
+    y = lineal(x, w, b)
+    got = [y, *torch.autograd.grad(y, (x, w, b), gy)]
+    d = lambda t: t.detach().double()
+    exact = [d(x) @ d(w).t() + d(b), d(gy) @ d(w), d(gy).t() @ d(x), d(gy).sum(0)]
+    for o, e in zip(got, exact):
+        assert _rel(o, e) <= tol
+
+
+def test_weight_gradient_in_a_graph():
+    """The split product replayed several times, with other work between the replays."""
+    g = torch.Generator(device='cuda').manual_seed(1)
+    a, b = torch.randn(4100, 96, generator=g, device='cuda'), torch.randn(4100, 64, generator=g, device='cuda')
+    ref = weight_grad(a, b, True)
+    lado = torch.cuda.Stream()
+    lado.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(lado):
+        weight_grad(a, b, True)
+    torch.cuda.current_stream().wait_stream(lado)
+    grafo = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(grafo):
+        out = weight_grad(a, b, True)
+    for _ in range(4):
+        for t in out:
+            t.fill_(-1.0)
+        grafo.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(x, y) for x, y in zip(out, ref))
+        gemm(a, True, b, False)
