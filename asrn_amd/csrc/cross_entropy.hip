@@ -2,12 +2,15 @@
 // reference's F.cross_entropy(logits.float(), y, ignore_index) does (asrn/nucleo.py:1108), without the fp32 copy of
 // the logits it makes.
 //
-//   k_ce_fwd  one workgroup per row: the row's max, then the sum of exp(x - max) (the row is read twice; the second
-//             read comes from L2), lse = max + log(sum); loss = lse - x[target] (0 for an ignored row, NaN for a
-//             target outside [0, V)).
+//   k_ce_fwd  one workgroup per row: the row's max, then the sum of exp(x - max), lse = max + log(sum); loss = lse -
+//             x[target] (0 for an ignored row, NaN for a target outside [0, V)). HBM-bound: a row of up to 65,536 bf16 or
+//             32,768 fp32 logits is read once and stays packed in registers between the two sums, every load in flight
+//             at once (8192 rows of 32,768 bf16: 164 us reading it twice); a longer one is read twice, the
+//             second time from L2. Up to 2,048 vectors of 16 bytes a row takes 256 threads, so that 8 rows share a CU
+//             and one row's loads run under another's sums; a longer one 1,024.
+//   k_ce_reduce  the rows' mean or sum and the count of rows not ignored, one workgroup, in a fixed order.
 //   k_ce_bwd  one workgroup per row: d logits = (exp(x - lse) - [v == target]) * scale, in the logits' dtype (bf16
 //             rounded to nearest even, as the cast back from fp32 rounds); an ignored row's gradient is 0.
-// The mean over the rows that are not ignored is left to the caller (a fixed-order sum of the per-row losses).
 #include <math.h>
 
 #include "common.h"
@@ -79,6 +82,7 @@ __device__ __forceinline__ void sweep_row(const void* logits, int64_t ld, int64_
 // max that keeps a NaN (fmaxf drops it; torch's max propagates it)
 __device__ __forceinline__ float nan_max(float a, float b) { return (a != a || b != b) ? NAN : fmaxf(a, b); }
 
+template <int THREADS>
 __device__ __forceinline__ float block_reduce(float x, float* red, bool is_max) {
   const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x >> 6;
 #pragma unroll
@@ -89,23 +93,64 @@ __device__ __forceinline__ float block_reduce(float x, float* red, bool is_max) 
   if (lane == 0) red[wave] = x;
   __syncthreads();
   float r = red[0];
-  for (int w = 1; w < kCeWaves; ++w) r = is_max ? nan_max(r, red[w]) : r + red[w];   // in wave order
+  for (int w = 1; w < THREADS / kWave; ++w) r = is_max ? nan_max(r, red[w]) : r + red[w];   // in wave order
   __syncthreads();
   return r;
 }
 
-template <bool B16>
-__global__ __launch_bounds__(kCeThreads) void k_ce_fwd(const void* logits, int64_t ld, const int64_t* target,
-                                                       int64_t V, int64_t ignore, float* lse, float* loss) {
-  __shared__ float red[kCeWaves];
+// the 8 bf16 or 4 fp32 values of a 16-byte vector
+template <bool B16, class F>
+__device__ __forceinline__ void each_of(const uint4& q, F f) {
+  const uint32_t w[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    if constexpr (B16) {
+      f(__uint_as_float(w[k] << 16));
+      f(__uint_as_float(w[k] & 0xffff0000u));
+    } else {
+      f(__uint_as_float(w[k]));
+    }
+  }
+}
+
+// NV: 16-byte vectors of the row a thread holds (0: the row is read twice instead)
+template <bool B16, int NV, int THREADS>
+__global__ __launch_bounds__(THREADS) void k_ce_fwd(const void* logits, int64_t ld, const int64_t* target,
+                                                    int64_t V, int64_t ignore, float* lse, float* loss) {
+  __shared__ float red[THREADS / kWave];
   const int64_t row = blockIdx.x;
-  float m = -INFINITY;
-  sweep_row<B16>(logits, ld, row, V, [&](int64_t, float x) { m = nan_max(m, x); });
-  const float mx = block_reduce(m, red, true);
-  float s = 0.f;
-  sweep_row<B16>(logits, ld, row, V, [&](int64_t, float x) { s += __expf(x - mx); });
-  const float tot = block_reduce(s, red, false);
-  if (threadIdx.x == 0) {
+  const int tid = threadIdx.x;
+  constexpr int E = B16 ? 8 : 4;
+  float m = -INFINITY, s = 0.f, mx;
+  if constexpr (NV > 0) {
+    const char* r = reinterpret_cast<const char*>(logits) + row * ld * (16 / E);
+    const int nvec = (int)(V / E);
+    uint4 q[NV];
+#pragma unroll
+    for (int u = 0; u < NV; ++u) {                 // lanes past the row read its first vector, not used
+      const int v = tid + u * THREADS;
+      q[u] = nvec > 0 ? reinterpret_cast<const uint4*>(r)[v < nvec ? v : 0] : make_uint4(0u, 0u, 0u, 0u);
+    }
+    const int tail = E * nvec + tid;               // V % E elements, one a thread
+    float xt = 0.f;
+    if (tail < V)
+      xt = B16 ? bf16_to_f32(reinterpret_cast<const uint16_t*>(r)[tail]) : reinterpret_cast<const float*>(r)[tail];
+#pragma unroll
+    for (int u = 0; u < NV; ++u)
+      if (tid + u * THREADS < nvec) each_of<B16>(q[u], [&](float x) { m = nan_max(m, x); });
+    if (tail < V) m = nan_max(m, xt);
+    mx = block_reduce<THREADS>(m, red, true);
+#pragma unroll
+    for (int u = 0; u < NV; ++u)
+      if (tid + u * THREADS < nvec) each_of<B16>(q[u], [&](float x) { s += __expf(x - mx); });
+    if (tail < V) s += __expf(xt - mx);
+  } else {
+    sweep_row<B16>(logits, ld, row, V, [&](int64_t, float x) { m = nan_max(m, x); });
+    mx = block_reduce<THREADS>(m, red, true);
+    sweep_row<B16>(logits, ld, row, V, [&](int64_t, float x) { s += __expf(x - mx); });
+  }
+  const float tot = block_reduce<THREADS>(s, red, false);
+  if (tid == 0) {
     const float l = mx + __logf(tot);
     lse[row] = l;
     const int64_t t = target[row];
@@ -119,6 +164,36 @@ __global__ __launch_bounds__(kCeThreads) void k_ce_fwd(const void* logits, int64
   }
 }
 
+// out = the sum of the rows' losses (mean: over the count of rows not ignored, NaN when there is none); divisor = that
+// count (1 for the sum): what the gradient is divided by
+__global__ __launch_bounds__(kCeThreads) void k_ce_reduce(const float* loss, const int64_t* target, int64_t rows,
+                                                          int64_t ignore, int mean, float* out, float* divisor) {
+  __shared__ float red[kCeWaves];
+  float s = 0.f, n = 0.f;                          // counts below 2^24 a thread: exact
+  for (int64_t r0 = threadIdx.x; r0 < rows; r0 += 8 * kCeThreads) {
+    float l[8];
+    int64_t t[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int64_t r = r0 + u * kCeThreads, rc = r < rows ? r : rows - 1;
+      l[u] = loss[rc];
+      t[u] = target[rc];
+    }
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      if (r0 + u * kCeThreads < rows) {
+        s += l[u];
+        n += t[u] != ignore ? 1.f : 0.f;
+      }
+  }
+  const float total = block_reduce<kCeThreads>(s, red, false);
+  const float count = block_reduce<kCeThreads>(n, red, false);
+  if (threadIdx.x == 0) {
+    *out = mean ? total / count : total;
+    *divisor = mean ? count : 1.f;
+  }
+}
+
 // one output element: (exp(x - lse) - [v == t]) * scale, 0 for an ignored row
 __device__ __forceinline__ float ce_grad(float x, int64_t v, int64_t t, float l, float sc, bool skip) {
   return skip ? 0.f : (__expf(x - l) - (v == t ? 1.f : 0.f)) * sc;
@@ -127,12 +202,13 @@ __device__ __forceinline__ float ce_grad(float x, int64_t v, int64_t t, float l,
 template <bool B16>
 __global__ __launch_bounds__(kCeThreads) void k_ce_bwd(const void* logits, int64_t ld, const int64_t* target,
                                                        const float* lse, int64_t V, int64_t ignore,
-                                                       const float* scale, void* dlogits, int64_t ldd) {
+                                                       const float* scale, const float* count, void* dlogits,
+                                                       int64_t ldd) {
   const int tid = threadIdx.x;
   const int64_t row = blockIdx.x;
   const int64_t t = target[row];
   const bool skip = t == ignore;
-  const float l = lse[row], sc = *scale;
+  const float l = lse[row], sc = count ? *scale / *count : *scale;
   if constexpr (B16) {                             // 8 elements per 16-byte load and store
     const uint16_t* r = reinterpret_cast<const uint16_t*>(logits) + row * ld;
     uint16_t* o = reinterpret_cast<uint16_t*>(dlogits) + row * ldd;
@@ -199,32 +275,56 @@ static int ce_check(const void* logits, int32_t bf16, int64_t ld, int64_t rows, 
 
 using namespace asrn;
 
+// the forward's registers: vectors a thread holds, by the row's length
+template <bool B16>
+static void launch_ce_fwd(const void* logits, int64_t ld, const int64_t* target, int64_t rows, int64_t V,
+                          int64_t ignore, float* lse, float* loss, hipStream_t st) {
+  const int64_t nvec = V / (B16 ? 8 : 4);
+  const dim3 grid((unsigned)rows);
+#define ASRN_CE(NV, TH) hipLaunchKernelGGL((k_ce_fwd<B16, NV, TH>), grid, dim3(TH), 0, st, logits, ld, target, V, \
+                                           ignore, lse, loss)
+  if (nvec <= 256) ASRN_CE(1, 256);
+  else if (nvec <= 512) ASRN_CE(2, 256);
+  else if (nvec <= 1024) ASRN_CE(4, 256);
+  else if (nvec <= 2048) ASRN_CE(8, 256);
+  else if (nvec <= 4 * kCeThreads) ASRN_CE(4, kCeThreads);
+  else if (nvec <= 8 * kCeThreads) ASRN_CE(8, kCeThreads);
+  else ASRN_CE(0, kCeThreads);
+#undef ASRN_CE
+}
+
 extern "C" int asrn_cross_entropy_fwd(const void* logits, int32_t logits_bf16, int64_t ld, const int64_t* target,
                                       int64_t rows, int64_t V, int64_t ignore_index, float* lse, float* loss,
                                       void* stream) {
   if (ce_check(logits, logits_bf16, ld, rows, V, "asrn_cross_entropy_fwd")) return 1;
   if (rows == 0) return 0;
-  if (logits_bf16)
-    hipLaunchKernelGGL(k_ce_fwd<true>, dim3((unsigned)rows), dim3(kCeThreads), 0, (hipStream_t)stream, logits, ld,
-                       target, V, ignore_index, lse, loss);
-  else
-    hipLaunchKernelGGL(k_ce_fwd<false>, dim3((unsigned)rows), dim3(kCeThreads), 0, (hipStream_t)stream, logits, ld,
-                       target, V, ignore_index, lse, loss);
+  if (logits_bf16) launch_ce_fwd<true>(logits, ld, target, rows, V, ignore_index, lse, loss, (hipStream_t)stream);
+  else launch_ce_fwd<false>(logits, ld, target, rows, V, ignore_index, lse, loss, (hipStream_t)stream);
   return check_launch("asrn_cross_entropy_fwd");
+}
+
+extern "C" int asrn_cross_entropy_reduce(const float* loss, const int64_t* target, int64_t rows, int64_t ignore_index,
+                                         int32_t mean, float* out, float* count, void* stream) {
+  ASRN_REQUIRE(rows >= 0 && rows < (int64_t(1) << 31), "asrn_cross_entropy_reduce: bad row count %lld",
+               (long long)rows);
+  hipLaunchKernelGGL(k_ce_reduce, dim3(1), dim3(kCeThreads), 0, (hipStream_t)stream, loss, target, rows, ignore_index,
+                     mean ? 1 : 0, out, count);
+  return check_launch("asrn_cross_entropy_reduce");
 }
 
 extern "C" int asrn_cross_entropy_bwd(const void* logits, int32_t logits_bf16, int64_t ld, const int64_t* target,
                                       const float* lse, int64_t rows, int64_t V, int64_t ignore_index,
-                                      const float* scale, void* dlogits, int64_t ldd, void* stream) {
+                                      const float* scale, const float* count, void* dlogits, int64_t ldd,
+                                      void* stream) {
   if (ce_check(logits, logits_bf16, ld, rows, V, "asrn_cross_entropy_bwd")) return 1;
   ASRN_REQUIRE(ldd >= V && ldd % (logits_bf16 ? 8 : 4) == 0 && ((uintptr_t)dlogits & 15) == 0,
                "asrn_cross_entropy_bwd: the gradient needs a row stride >= V that keeps 16-byte aligned rows");
   if (rows == 0) return 0;
   if (logits_bf16)
     hipLaunchKernelGGL(k_ce_bwd<true>, dim3((unsigned)rows), dim3(kCeThreads), 0, (hipStream_t)stream, logits, ld,
-                       target, lse, V, ignore_index, scale, dlogits, ldd);
+                       target, lse, V, ignore_index, scale, count, dlogits, ldd);
   else
     hipLaunchKernelGGL(k_ce_bwd<false>, dim3((unsigned)rows), dim3(kCeThreads), 0, (hipStream_t)stream, logits, ld,
-                       target, lse, V, ignore_index, scale, dlogits, ldd);
+                       target, lse, V, ignore_index, scale, count, dlogits, ldd);
   return check_launch("asrn_cross_entropy_bwd");
 }

@@ -1242,8 +1242,8 @@ def norma_pendiente(ln, previo, avance=None):
 class CrossEntropy(torch.autograd.Function):
     """F.cross_entropy(logits.float().reshape(-1, V), target.reshape(-1), ignore_index, reduction) for 'mean' and
     'sum' (asrn/nucleo.py:1108): asrn_cross_entropy_fwd/bwd compute it in fp32 from fp32 or bf16 logits as they are
-    (no fp32 copy), and the gradient comes back in the logits' dtype. The rows are reduced here: the mean divides the
-    summed row losses by the count of rows not ignored (NaN when there is none, as PyTorch gives)."""
+    (no fp32 copy), and the gradient comes back in the logits' dtype. asrn_cross_entropy_reduce sums the rows: the mean
+    divides by the count of rows not ignored (NaN when there is none, as PyTorch gives)."""
 
     @staticmethod
     def forward(ctx, logits, target, ignore_index, reduction):
@@ -1269,29 +1269,25 @@ class CrossEntropy(torch.autograd.Function):
         per = torch.empty((rows,), dtype=torch.float32, device=dev)
         call('asrn_cross_entropy_fwd', ptr(x), int(bf16), ld, ptr(t), rows, V, int(ignore_index), ptr(lse), ptr(per),
              stream_of(dev))
-        total = per.sum()
-        if reduction == 'mean':
-            count = (t != ignore_index).sum().to(torch.float32)
-            out = total / count
-        else:
-            count = None
-            out = total
-        ctx.save_for_backward(x, t, lse, count if count is not None else total)
-        ctx.meta = (int(ignore_index), reduction, logits.shape, logits.dtype, bf16)
+        out = torch.empty((), dtype=torch.float32, device=dev)
+        count = torch.empty((), dtype=torch.float32, device=dev)       # what the gradient is divided by
+        call('asrn_cross_entropy_reduce', ptr(per), ptr(t), rows, int(ignore_index), int(reduction == 'mean'), ptr(out),
+             ptr(count), stream_of(dev))
+        ctx.save_for_backward(x, t, lse, count)
+        ctx.meta = (int(ignore_index), logits.shape, logits.dtype, bf16)
         return out
 
     @staticmethod
     def backward(ctx, g):
         x, t, lse, count = ctx.saved_tensors
-        ignore_index, reduction, shape, dtype, bf16 = ctx.meta
+        ignore_index, shape, dtype, bf16 = ctx.meta
         rows, V = x.shape
         dev = x.device
-        scale = (g.float() / count) if reduction == 'mean' else g.float().reshape(())
-        scale = scale.reshape(1).contiguous()
+        scale = _c(g, torch.float32)
         ld = V + (-V % (8 if bf16 else 4))
         dx = torch.empty((rows, ld), dtype=x.dtype, device=dev)
         call('asrn_cross_entropy_bwd', ptr(x), int(bf16), x.stride(0), ptr(t), ptr(lse), rows, V, ignore_index,
-             ptr(scale), ptr(dx), ld, stream_of(dev))
+             ptr(scale), ptr(count), ptr(dx), ld, stream_of(dev))
         return dx[:, :V].reshape(shape).to(dtype), None, None, None
 
 

@@ -561,14 +561,18 @@ int asrn_block_finish_norm(const float* prev_h1, const float* prev_b2, const flo
  * training loop (asrn/nucleo.py:1108, 2301): the same fp32 arithmetic on fp32 or bf16 logits (logits_bf16), without
  * the fp32 copy of the logits. logits (rows, V) with row stride ld (16-byte aligned rows), target (rows) int64.
  * fwd: lse (rows) = logsumexp of the row, loss (rows) = lse - logits[target] (0 where target == ignore_index, NaN
- * for a target outside [0, V)); the caller reduces the rows (mean over the rows not ignored, or sum).
- * bwd: dlogits (rows, V), row stride ldd, in the logits' dtype = (softmax - onehot(target)) * *scale (scale a device
- * float: d loss / count for the mean), 0 for ignored rows; bf16 rounded to nearest even. */
+ * for a target outside [0, V)). reduce: *out = the sum of the rows' losses, over the count of rows not ignored with
+ * mean (NaN when there is none); *count = that count (1 without mean).
+ * bwd: dlogits (rows, V), row stride ldd, in the logits' dtype = (softmax - onehot(target)) * *scale / *count (device
+ * floats: the loss's gradient and reduce's count, which may be null), 0 for ignored rows; bf16 rounded to nearest
+ * even. */
 int asrn_cross_entropy_fwd(const void* logits, int32_t logits_bf16, int64_t ld, const int64_t* target, int64_t rows,
                            int64_t V, int64_t ignore_index, float* lse, float* loss, void* stream);
+int asrn_cross_entropy_reduce(const float* loss, const int64_t* target, int64_t rows, int64_t ignore_index,
+                              int32_t mean, float* out, float* count, void* stream);
 int asrn_cross_entropy_bwd(const void* logits, int32_t logits_bf16, int64_t ld, const int64_t* target,
                            const float* lse, int64_t rows, int64_t V, int64_t ignore_index, const float* scale,
-                           void* dlogits, int64_t ldd, void* stream);
+                           const float* count, void* dlogits, int64_t ldd, void* stream);
 
 /* ---- the model's local block: the causal convolution's columns ----------------------------------------------
  * Replaces F.pad + unfold + reshape of the 'conv' BloqueLocal's convolution (asrn/nucleo.py:969-1014, nn.Conv1d over
