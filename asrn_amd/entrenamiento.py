@@ -145,8 +145,12 @@ class PasoGrafado:
             logits = self.modelo(self.x)
         perdida = entropia(logits, self.y)
         perdida.backward()
-        norma = torch.nn.utils.clip_grad_norm_(self.params, self.recorte)
-        salto = (~(torch.isfinite(perdida) & torch.isfinite(norma))).float()
+        recorte = ops.recortar_gradientes(self.params, self.recorte, perdida)
+        if recorte is None:
+            norma = torch.nn.utils.clip_grad_norm_(self.params, self.recorte)
+            salto = (~(torch.isfinite(perdida) & torch.isfinite(norma))).float()
+        else:
+            norma, salto = recorte
         if self.opt.param_groups[0].get('fused'):
             self.opt.found_inf = salto               # read by the fused kernel on the device: no host sync
             try:

@@ -1300,6 +1300,31 @@ def cross_entropy(logits, target, ignore_index=-100, reduction='mean'):
 
 
 # ---------------------------------------------------------------------------------------------------------------------
+# the training step's gradient clipping
+# ---------------------------------------------------------------------------------------------------------------------
+
+@torch.no_grad()
+def recortar_gradientes(params, maximo, perdida):
+    """clip_grad_norm_(params, maximo) and the step's check in three launches (asrn_clip_gradients): the gradients are
+    scaled in place; returns (their norm, 1.0 when the loss or the norm is not finite else 0.0) as device scalars.
+    None when a gradient or the loss is not a contiguous fp32 tensor on one GPU."""
+    gs = [p.grad for p in params if p.grad is not None]
+    if not gs or not perdida.is_cuda or not all(
+            g.device == perdida.device and g.dtype == torch.float32 and g.layout == torch.strided and g.is_contiguous()
+            for g in gs) or perdida.dtype != torch.float32 or perdida.numel() != 1:
+        return None
+    dev, n = perdida.device, len(gs)
+    sizes = (ctypes.c_int64 * n)(*[g.numel() for g in gs])
+    ptrs = (ctypes.c_void_p * n)(*[g.data_ptr() for g in gs])
+    wsb = query('asrn_clip_gradients_workspace', n, sizes)
+    ws = torch.empty((wsb,), dtype=torch.uint8, device=dev)
+    norma, salto = (torch.empty((), dtype=torch.float32, device=dev) for _ in range(2))
+    call('asrn_clip_gradients', n, ptrs, sizes, float(maximo), ptr(perdida), ptr(norma), ptr(salto), ptr(ws), wsb,
+         stream_of(dev))
+    return norma, salto
+
+
+# ---------------------------------------------------------------------------------------------------------------------
 # the local block's convolution window
 # ---------------------------------------------------------------------------------------------------------------------
 

@@ -574,6 +574,15 @@ int asrn_cross_entropy_bwd(const void* logits, int32_t logits_bf16, int64_t ld, 
                            const float* lse, int64_t rows, int64_t V, int64_t ignore_index, const float* scale,
                            const float* count, void* dlogits, int64_t ldd, void* stream);
 
+/* ---- the training step's gradient clipping -----------------------------------------------------------------------
+ * Replaces clip_grad_norm_ and the non-finite test of PasoGrafado (asrn/nucleo.py:2253-2343): over n fp32 gradients of
+ * sizes[i] values (host arrays of device addresses and sizes), *norm = their 2-norm, every gradient scaled in place by
+ * min(1, max_norm / (*norm + 1e-6)), *skip = 1 when *loss or *norm is not finite, else 0. workspace:
+ * asrn_clip_gradients_workspace bytes, 8-byte aligned. */
+int64_t asrn_clip_gradients_workspace(int32_t n, const int64_t* sizes);
+int asrn_clip_gradients(int32_t n, float* const* grads, const int64_t* sizes, float max_norm, const float* loss,
+                        float* norm, float* skip, void* workspace, int64_t workspace_bytes, void* stream);
+
 /* ---- the model's local block: the causal convolution's columns ----------------------------------------------
  * Replaces F.pad + unfold + reshape of the 'conv' BloqueLocal's convolution (asrn/nucleo.py:969-1014, nn.Conv1d over
  * the left-padded sequence) and the cast of those columns to the autocast dtype. fwd: z (B, L, d) fp32, row stride
