@@ -194,7 +194,7 @@ class ModeloASRN(nn.Module):
     def estado(self, x):
         """The last block's output, before ln_f and the head: (B, L, d)."""
         revisar_precision(self)
-        E = self.emb(x)
+        E = ops.incrustar(self.emb, x)
         recalcular = self.training and torch.is_grad_enabled()
         ck_bloque = recalcular and self.checkpoint == 'todo'
         ck_capa = recalcular and self.checkpoint != 'no'

@@ -1300,6 +1300,44 @@ def cross_entropy(logits, target, ignore_index=-100, reduction='mean'):
 
 
 # ---------------------------------------------------------------------------------------------------------------------
+# the embedding
+# ---------------------------------------------------------------------------------------------------------------------
+
+FICHAS_INCRUSTAR = 4096      # most tokens asrn_embedding_bwd takes; past them torch's sort-based backward runs
+
+
+class Incrustar(torch.autograd.Function):
+    """emb.weight[x] with the gradient from asrn_embedding_bwd: the same sums in position order, deterministic."""
+
+    @staticmethod
+    def forward(ctx, w, x):
+        ctx.save_for_backward(x)
+        ctx.forma = w.shape
+        return F.embedding(x, w)
+
+    @staticmethod
+    def backward(ctx, g):
+        x, = ctx.saved_tensors
+        V, d = ctx.forma
+        dw = torch.empty((V, d), dtype=torch.float32, device=g.device)
+        gc, xc = _c(g, torch.float32), x.contiguous()
+        call('asrn_embedding_bwd', ptr(gc), ptr(xc), xc.numel(), V, d, ptr(dw), stream_of(g.device))
+        return dw, None
+
+
+def incrustar(emb, x):
+    """emb(x); for a plain fp32 nn.Embedding in training on up to FICHAS_INCRUSTAR int64 tokens, with asrn_embedding_bwd
+    as its backward."""
+    w = emb.weight
+    if (w.is_cuda and x.device == w.device and x.dtype == torch.int64 and w.dtype == torch.float32 and w.requires_grad
+            and torch.is_grad_enabled() and 1 <= x.numel() <= FICHAS_INCRUSTAR and type(emb) is torch.nn.Embedding
+            and emb.padding_idx is None and emb.max_norm is None and not emb.scale_grad_by_freq and not emb.sparse
+            and not emb._forward_hooks and not emb._forward_pre_hooks and not emb._backward_hooks):
+        return Incrustar.apply(w, x)
+    return emb(x)
+
+
+# ---------------------------------------------------------------------------------------------------------------------
 # the training step's gradient clipping
 # ---------------------------------------------------------------------------------------------------------------------
 

@@ -574,6 +574,11 @@ int asrn_cross_entropy_bwd(const void* logits, int32_t logits_bf16, int64_t ld, 
                            const float* lse, int64_t rows, int64_t V, int64_t ignore_index, const float* scale,
                            const float* count, void* dlogits, int64_t ldd, void* stream);
 
+/* ---- the embedding's gradient -------------------------------------------------------------------------------------
+ * Replaces nn.Embedding's backward (asrn/nucleo.py:1047-1125) for 1 <= n <= 4,096 tokens: dW (V, d) = for every row v
+ * the sum of dE's rows (n, d), fp32, over the positions i with ids[i] == v, in order (0 where there is none). */
+int asrn_embedding_bwd(const float* dE, const int64_t* ids, int64_t n, int64_t V, int32_t d, float* dW, void* stream);
+
 /* ---- the training step's gradient clipping -----------------------------------------------------------------------
  * Replaces clip_grad_norm_ and the non-finite test of PasoGrafado (asrn/nucleo.py:2253-2343): over n fp32 gradients of
  * sizes[i] values (host arrays of device addresses and sizes), *norm = their 2-norm, every gradient scaled in place by

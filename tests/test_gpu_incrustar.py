@@ -1,0 +1,26 @@
+"""asrn_embedding_bwd (ops.incrustar) against torch's embedding gradient in float64: vocabularies and widths off the
+workgroup's 16 rows and 64 columns, one token, one token everywhere (its whole list in one workgroup), the longest
+batch. fp32 sums of up to n rows: 2^-24 sqrt(n) relative to the sum of magnitudes."""
+import pytest
+import torch
+
+from asrn_amd import ops
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize('B,L,V,d,uno', [(1, 1, 1, 4, False), (3, 333, 257, 68, False), (2, 2048, 16, 64, True),
+                                         (8, 512, 1000, 192, False), (1, 511, 8000, 100, False)])
+def test_matches_torch(B, L, V, d, uno):
+    g = torch.Generator(device='cuda').manual_seed(V)
+    emb = torch.nn.Embedding(V, d).cuda()
+    x = torch.randint(0, V, (B, L), generator=g, device='cuda')
+    if uno:
+        x.fill_(V - 1)
+    gy = torch.randn(B, L, d, generator=g, device='cuda')
+    y = ops.incrustar(emb, x)
+    assert torch.equal(y, emb(x))
+    dw, = torch.autograd.grad(y, emb.weight, gy)
+    ref = torch.zeros(V, d, dtype=torch.float64, device='cuda').index_add_(0, x.reshape(-1), gy.double().reshape(-1, d))
+    mag = torch.zeros_like(ref).index_add_(0, x.reshape(-1), gy.double().abs().reshape(-1, d))
+    assert bool(((dw.double() - ref).abs() <= 2.0 ** -24 * (B * L) ** 0.5 * mag + 1e-30).all())
