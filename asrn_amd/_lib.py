@@ -30,6 +30,7 @@ SIGNATURES = {
                             + [_F32, _F32, _I64, _I32, _I64, _I32] + [_P] * 11),
     'asrn_scan_workspace': (_I64, [_I64, _I64]),
     'asrn_clock_scan': (ctypes.c_int, [_P, _P, _I64, _I64, _I32, _P, _I64, _P]),
+    'asrn_clock_bwd': (ctypes.c_int, [_P] * 5 + [_I64, _I64, _P, _P, _P, _I64, _P]),
     'asrn_ngram_sort_workspace': (_I64, [_I64, _I64, _I32]),
     'asrn_ngram_sort': (ctypes.c_int, [_P, _P, _I64, _I64, _I32, _P, _P, _P, _P, _P, _P, _I64, _P]),
     'asrn_scan_fwd': (ctypes.c_int, [_P, _P, _P, _I64, _I64, _P, _I64, _P]),
@@ -42,9 +43,9 @@ SIGNATURES = {
     'asrn_streak_fwd': (ctypes.c_int, [_P, _P, _P, _I64, _I64, _I32, _P, _P, _I64, _P]),
     'asrn_streak_bwd': (ctypes.c_int, [_P, _P, _P, _P, _P, _I64, _I64, _I32, _P, _P, _P, _I64, _P]),
     'asrn_repetition_workspace': (_I64, [_I64, _I64, _I32]),
-    'asrn_repetition_fwd': (ctypes.c_int, [_P] * 8 + [_I64, _I64, _I32] + [_P] * 4 + [_I64, _P]),
+    'asrn_repetition_fwd': (ctypes.c_int, [_P] * 8 + [_I32, _I64, _I64, _I32] + [_P] * 4 + [_I64, _P]),
     'asrn_repetition_bwd_workspace': (_I64, [_I64, _I64, _I32]),
-    'asrn_repetition_bwd': (ctypes.c_int, [_P] * 13 + [_I64, _I64, _I32] + [_P] * 6 + [_I64, _P]),
+    'asrn_repetition_bwd': (ctypes.c_int, [_P] * 11 + [_I32, _P, _P, _I64, _I64, _I32] + [_P] * 6 + [_I64, _P]),
     'asrn_context_fwd': (ctypes.c_int, [_P] * 5 + [_I64, _I32] + [_F32] * 3 + [_P] * 5),
     'asrn_context_bwd_workspace': (_I64, [_I64, _I32]),
     'asrn_context_bwd': (ctypes.c_int, [_P] * 5 + [_I64, _I32] + [_F32] * 2 + [_P] * 2 + [_I64, _I32] + [_P] * 7

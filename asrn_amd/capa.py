@@ -289,12 +289,14 @@ class CapaASRNEstable(nn.Module):
     def _repeticion(self, sig, beta, Bt, log_alfa, partes=None, ngram=None):
         """vistos, hawkes (B, L, n) and racha (B, L) (asrn/estable.py:304-321); ngram: ops.ngram_sort(sig, ...) when
         it already ran."""
-        kappa, kappa_r = self._kappas()
+        # the rates from their logarithms in the scans' kernels, unless a floor holds them
+        logs = self.protecciones.kappa_min is None
+        kappa, kappa_r = (self.log_kappa, self.log_kappa_racha) if logs else self._kappas()
         if ngram is None:
             with torch.no_grad():
                 ngram = ops.ngram_sort(sig, self.c_vistos, self.vistos)
         claves, order, rep, rank_k, vistos = ngram
-        hawkes, racha = ops.Repeticion.apply(Bt, log_alfa, kappa, beta, kappa_r, order, rep, rank_k, vistos)
+        hawkes, racha = ops.Repeticion.apply(Bt, log_alfa, kappa, beta, kappa_r, order, rep, rank_k, vistos, logs)
         if partes is not None:
             partes.update(claves=claves, orden_k=order, repetido=rep)
         return {'vistos': vistos, 'hawkes': hawkes, 'racha': racha}
@@ -398,7 +400,7 @@ class CapaASRNEstable(nn.Module):
             w_salida = ops.SmallMatmul.apply(self.o.weight, self.v.weight)
             Qc, Kc, beta, log_alfa, h = self._contexto(h, con_h=True, pesos=pesos)
             # the clock: fp64 (reloj_64), or the core layer's fp32 clock, each sum rounded to fp32 (kept in fp64)
-            Bt = ops.ClockScan.apply(beta, not self.protecciones.reloj_64)
+            Bt, Bt_rep, log_alfa, la_rep, beta = ops.Reloj.apply(beta, log_alfa, not self.protecciones.reloj_64)
             contexto_listo = torch.cuda.Event()
             contexto_listo.record(lado)
             if ngramas is None:
@@ -406,7 +408,7 @@ class CapaASRNEstable(nn.Module):
                     ngram = ops.ngram_sort(sig, self.c_vistos, self.vistos)
             else:
                 ngram = ngramas[1:]
-            rep = self._repeticion(sig, beta, Bt, log_alfa, partes, ngram)
+            rep = self._repeticion(sig, beta, Bt_rep, la_rep, partes, ngram)
         if pesos is not None:
             pesos['Wq'].record_stream(lado)            # made here, used there: not reused before both are done
         acc = self._acumular(E, Qc, Kc, Bt, log_alfa, sig, partes, pesos,

@@ -210,10 +210,12 @@ struct PlainBwd {
 struct HawkesCommon {
   const int32_t* order; const uint8_t* rep; const double* Bt; const float* la; const float* kappa;
   int64_t L; int n;
+  int logs = 0;                                  // kappa holds the rates' logarithms
+  __device__ __forceinline__ float rate(int j) const { return logs ? expf(kappa[j]) : kappa[j]; }
   __device__ __forceinline__ float step(int j, double diff, float* dB, bool* pass) const {
     *dB = (float)(diff < 0.0 ? 0.0 : diff);
     *pass = diff >= 0.0;                         // the clamp passes the gradient
-    return expf(-kappa[j] * *dB);
+    return expf(-rate(j) * *dB);
   }
 };
 
@@ -287,7 +289,7 @@ struct HawkesBwd : HawkesCommon {
     if (x.a != 0.f) {
       const float ga = lam * (x.Sprev + x.alfa);   // b_i = a_i alfa_{i-1}
       const float gz = ga * x.a;                   // d a / d z = a (z = -kappa dB)
-      g = x.pass ? -kappa[j] * gz : 0.f;
+      g = x.pass ? -rate(j) * gz : 0.f;
       acc += gz * -x.dB;
       w = lam * x.a;                               // d L / d alfa_{i-1}
     }
@@ -297,10 +299,25 @@ struct HawkesBwd : HawkesCommon {
   __device__ void reduce(int row, float s) const { dkappa[row] = s; }
 };
 
+// What the last workgroup of k_hawkes_bwd_finish does when `rows` is given: the rates' gradients, summed over the batch
+// rows in order (rows: B n Hawkes sums, then B streak sums), times the rates when they came as logarithms
+struct RateGrads { const float* rows; const float* kappa; const float* kappa_r; float* dkappa; float* dkappa_r; int logs; };
+
 // per text position: dBt = sum_j (gdB_j[i] - gdB_j[i+1]) in fp64, dlog_alfa = alfa_t sum_j w_j[i+1]
 __global__ void k_hawkes_bwd_finish(const int32_t* __restrict__ rank_k, const float* __restrict__ gdB,
                                     const float* __restrict__ wa, const float* __restrict__ la, int64_t B, int64_t L,
-                                    int n, double* __restrict__ dBt, float* __restrict__ dla) {
+                                    int n, double* __restrict__ dBt, float* __restrict__ dla, RateGrads rg) {
+  if (rg.rows && blockIdx.x == gridDim.x - 1) {
+    const int j = threadIdx.x;
+    if (j <= n) {
+      const float* r = j < n ? rg.rows + j : rg.rows + B * n;
+      float s = 0.f;
+      for (int64_t b = 0; b < B; ++b) s += r[b * (j < n ? n : 1)];
+      const float* k = j < n ? rg.kappa + j : rg.kappa_r;
+      (j < n ? rg.dkappa + j : rg.dkappa_r)[0] = rg.logs ? s * expf(*k) : s;
+    }
+    return;
+  }
   const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= B * L) return;
   const int64_t bb = e / L, t = e % L;
@@ -321,9 +338,11 @@ __global__ void k_hawkes_bwd_finish(const int32_t* __restrict__ rank_k, const fl
 // ---- streak over the text (reference asrn/estable.py:319-320) -------------------------------------------------------
 struct StreakCommon {
   const float* vistos; const double* beta; const float* kappa_r; int64_t L; int n;
+  int logs = 0;
+  __device__ __forceinline__ float rate() const { return logs ? expf(kappa_r[0]) : kappa_r[0]; }
   __device__ float r_at(int row, int64_t t) const { return vistos[(row * L + t) * n + n - 1]; }
   __device__ float a_at(int row, int64_t t) const {
-    return r_at(row, t) * expf(-kappa_r[0] * (float)beta[row * L + t]);
+    return r_at(row, t) * expf(-rate() * (float)beta[row * L + t]);
   }
 };
 
@@ -355,7 +374,7 @@ struct StreakBwd : StreakCommon {
     const int64_t t = L - 1 - e;
     const float ga = t > 0 ? lam * x.rprev : 0.f;
     const float gz = ga * x.a;
-    dbeta[row * L + t] = (double)(gz * -kappa_r[0]);
+    dbeta[row * L + t] = (double)(gz * -rate());
     acc += gz * -x.beta;
   }
   __device__ void reduce(int row, float s) const { dkr[row] = s; }
@@ -373,6 +392,29 @@ struct ClockOp {
   __device__ Sum64 load(int row, int64_t e, Aux&) const { return {x[row * L + (reverse ? L - 1 - e : e)]}; }
   __device__ void store(int row, int64_t e, double v, float&, const Aux&) const {
     y[row * L + (reverse ? L - 1 - e : e)] = round32 ? (double)(float)v : v;
+  }
+  __device__ void reduce(int, float) const {}
+};
+
+// The clock's gradient with everything that joins it: dbeta = suffix sums of (g1 + g2) + add, and dla = l1 + l2 beside it
+// (any of them null: zero), so that the two users of the clock and of log alfa need no additions of their own.
+struct ClockBwd {
+  static constexpr bool kReduce = false;
+  static constexpr bool kOneLaunch = true;
+  using M = Sum64;
+  struct Aux { double add; float la; };
+  const double* g1; const double* g2; const double* add; const float* l1; const float* l2; double* dbeta; float* dla;
+  int64_t L;
+  __device__ Sum64 load(int row, int64_t e, Aux& x) const {
+    const int64_t i = row * L + L - 1 - e;
+    x.add = add ? add[i] : 0.0;
+    x.la = (l1 ? l1[i] : 0.f) + (l2 ? l2[i] : 0.f);
+    return {(g1 ? g1[i] : 0.0) + (g2 ? g2[i] : 0.0)};
+  }
+  __device__ void store(int row, int64_t e, double v, float&, const Aux& x) const {
+    const int64_t i = row * L + L - 1 - e;
+    dbeta[i] = v + x.add;
+    dla[i] = x.la;
   }
   __device__ void reduce(int, float) const {}
 };
@@ -487,6 +529,14 @@ extern "C" int asrn_clock_scan(const double* x, double* y, int64_t B, int64_t L,
   return launch_scan(op, B, L, workspace, workspace_bytes, stream, "asrn_clock_scan");
 }
 
+extern "C" int asrn_clock_bwd(const double* g1, const double* g2, const double* add, const float* l1, const float* l2,
+                              int64_t B, int64_t L, double* dbeta, float* dlog_alfa, void* workspace,
+                              int64_t workspace_bytes, void* stream) {
+  ASRN_REQUIRE(B >= 0 && L >= 0, "asrn_clock_bwd: bad sizes");
+  ClockBwd op{g1, g2, add, l1, l2, dbeta, dlog_alfa, L};
+  return launch_scan(op, B, L, workspace, workspace_bytes, stream, "asrn_clock_bwd");
+}
+
 extern "C" int asrn_scan_fwd(const float* a, const float* b, float* S, int64_t rows, int64_t N, void* workspace,
                              int64_t workspace_bytes, void* stream) {
   ASRN_REQUIRE(rows >= 0 && N >= 0, "asrn_scan_fwd: bad sizes");
@@ -579,7 +629,7 @@ extern "C" int asrn_hawkes_bwd(const int32_t* order, const uint8_t* repeated, co
   if (launch_scan(op, B * n, L, scan_ws, need - (scan_ws - (char*)workspace), stream, "asrn_hawkes_bwd")) return 1;
   const int threads = 256;
   hipLaunchKernelGGL(k_hawkes_bwd_finish, dim3((unsigned)((B * L + threads - 1) / threads)), dim3(threads), 0,
-                     (hipStream_t)stream, rank_k, gdB, wa, log_alfa, B, L, (int)n, dBt, dlog_alfa);
+                     (hipStream_t)stream, rank_k, gdB, wa, log_alfa, B, L, (int)n, dBt, dlog_alfa, RateGrads{});
   return check_launch("asrn_hawkes_bwd/finish");
 }
 
@@ -610,11 +660,12 @@ extern "C" int64_t asrn_repetition_workspace(int64_t B, int64_t L, int32_t n) {
 
 extern "C" int asrn_repetition_fwd(const int32_t* order, const uint8_t* repeated, const double* Bt,
                                    const float* log_alfa, const float* kappa, const float* vistos, const double* beta,
-                                   const float* kappa_r, int64_t B, int64_t L, int32_t n, float* hawkes,
+                                   const float* kappa_r, int32_t logs, int64_t B, int64_t L, int32_t n, float* hawkes,
                                    float* S_sorted, float* racha, void* workspace, int64_t workspace_bytes,
                                    void* stream) {
   ASRN_REQUIRE(B >= 0 && L >= 0 && n >= 1, "asrn_repetition_fwd: bad sizes");
   Both<HawkesFwd, StreakFwd> op;
+  op.a.logs = op.b.logs = logs ? 1 : 0;
   op.a.order = order; op.a.rep = repeated; op.a.Bt = Bt; op.a.la = log_alfa; op.a.kappa = kappa; op.a.L = L;
   op.a.n = n; op.a.hawkes = hawkes; op.a.S_sorted = S_sorted;
   op.b.vistos = vistos; op.b.beta = beta; op.b.kappa_r = kappa_r; op.b.L = L; op.b.n = n; op.b.racha = racha;
@@ -625,34 +676,38 @@ extern "C" int asrn_repetition_fwd(const int32_t* order, const uint8_t* repeated
 extern "C" int64_t asrn_repetition_bwd_workspace(int64_t B, int64_t L, int32_t n) {
   const int64_t scan = asrn_repetition_workspace(B, L, n);
   if (scan < 0) return -1;
-  return round_up(2 * B * L * n * (int64_t)sizeof(float)) + scan;
+  return round_up(2 * B * L * n * (int64_t)sizeof(float)) + round_up(B * (n + 1) * (int64_t)sizeof(float)) + scan;
 }
 
 extern "C" int asrn_repetition_bwd(const int32_t* order, const uint8_t* repeated, const int32_t* rank_k,
                                    const double* Bt, const float* log_alfa, const float* kappa, const float* S_sorted,
                                    const float* dhawkes, const float* vistos, const double* beta,
-                                   const float* kappa_r, const float* racha, const float* dracha, int64_t B,
-                                   int64_t L, int32_t n, double* dBt, float* dlog_alfa, float* dkappa,
+                                   const float* kappa_r, int32_t logs, const float* racha, const float* dracha,
+                                   int64_t B, int64_t L, int32_t n, double* dBt, float* dlog_alfa, float* dkappa,
                                    double* dbeta, float* dkappa_r, void* workspace, int64_t workspace_bytes,
                                    void* stream) {
   ASRN_REQUIRE(B >= 0 && L >= 0 && n >= 1, "asrn_repetition_bwd: bad sizes");
+  ASRN_REQUIRE(n < 256, "asrn_repetition_bwd: n=%d must be below 256", n);
   if (B == 0 || L == 0) return 0;
   const int64_t need = asrn_repetition_bwd_workspace(B, L, n);
   ASRN_REQUIRE(need >= 0, "asrn_repetition_bwd: rows x chunks must stay below 2^31");
   ASRN_REQUIRE(workspace != nullptr && workspace_bytes >= need, "asrn_repetition_bwd: workspace too small");
   float* gdB = (float*)workspace;
   float* wa = gdB + B * L * n;
-  char* scan_ws = (char*)workspace + round_up(2 * B * L * n * (int64_t)sizeof(float));
+  float* rows = (float*)((char*)workspace + round_up(2 * B * L * n * (int64_t)sizeof(float)));
+  char* scan_ws = (char*)rows + round_up(B * (n + 1) * (int64_t)sizeof(float));
   Both<HawkesBwd, StreakBwd> op;
   op.a.order = order; op.a.rep = repeated; op.a.Bt = Bt; op.a.la = log_alfa; op.a.kappa = kappa; op.a.L = L;
-  op.a.n = n; op.a.S_sorted = S_sorted; op.a.dh = dhawkes; op.a.gdB = gdB; op.a.wa = wa; op.a.dkappa = dkappa;
+  op.a.n = n; op.a.S_sorted = S_sorted; op.a.dh = dhawkes; op.a.gdB = gdB; op.a.wa = wa; op.a.dkappa = rows;
   op.b.vistos = vistos; op.b.beta = beta; op.b.kappa_r = kappa_r; op.b.L = L; op.b.n = n;
-  op.b.racha = racha; op.b.dr = dracha; op.b.dbeta = dbeta; op.b.dkr = dkappa_r;
+  op.b.racha = racha; op.b.dr = dracha; op.b.dbeta = dbeta; op.b.dkr = rows + B * n;
+  op.a.logs = op.b.logs = logs ? 1 : 0;
   op.ra = (int)(B * n);
   if (launch_scan(op, B * (n + 1), L, scan_ws, need - (scan_ws - (char*)workspace), stream, "asrn_repetition_bwd"))
     return 1;
   const int threads = 256;
-  hipLaunchKernelGGL(k_hawkes_bwd_finish, dim3((unsigned)((B * L + threads - 1) / threads)), dim3(threads), 0,
-                     (hipStream_t)stream, rank_k, gdB, wa, log_alfa, B, L, (int)n, dBt, dlog_alfa);
+  hipLaunchKernelGGL(k_hawkes_bwd_finish, dim3((unsigned)((B * L + threads - 1) / threads + 1)), dim3(threads), 0,
+                     (hipStream_t)stream, rank_k, gdB, wa, log_alfa, B, L, (int)n, dBt, dlog_alfa,
+                     RateGrads{rows, kappa, kappa_r, dkappa, dkappa_r, logs ? 1 : 0});
   return check_launch("asrn_repetition_bwd/finish");
 }

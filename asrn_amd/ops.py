@@ -100,9 +100,9 @@ def ngram_sort(sig, coef, n):
     keys = torch.empty((B, L, n), dtype=torch.float64, device=dev)
     order = torch.empty((B, n, L), dtype=I32, device=dev)
     rep = torch.empty((B, n, L), dtype=torch.uint8, device=dev)
-    buf = torch.zeros((2, B * n * L), dtype=I32, device=dev)   # one fill: every index read later is in range
+    buf = torch.empty((2, B * n * L), dtype=I32, device=dev)   # the sort writes every rank and flag
     rank_k = buf[0].view(B, n, L)
-    vistos = buf[1].view(torch.float32).view(B, L, n)              # int32 zeros are fp32 zeros
+    vistos = buf[1].view(torch.float32).view(B, L, n)
     wsb = query('asrn_ngram_sort_workspace', B, L, n)
     ws = torch.empty((max(wsb, 1),), dtype=torch.uint8, device=dev)
     call('asrn_ngram_sort', ptr(sig), ptr(coef), B, L, n, ptr(keys), ptr(order), ptr(rep), ptr(rank_k), ptr(vistos),
@@ -459,6 +459,34 @@ class ClockScan(torch.autograd.Function):
         return out, None
 
 
+class Reloj(torch.autograd.Function):
+    """ClockScan with the clock's, log alfa's and beta's two users apart: (Bt, Bt, log_alfa, log_alfa, beta), the
+    repeated ones aliases, for the candidates and for the repetition scans (beta for the streak). The backward sums
+    their gradients in the suffix scan's launch (asrn_clock_bwd)."""
+
+    @staticmethod
+    def forward(ctx, beta, log_alfa, reloj32=False):
+        dev = _dev(beta)
+        x, la = _c(beta, torch.float64), _c(log_alfa, torch.float32)
+        B, L = x.shape
+        y = torch.empty((B * L,), dtype=torch.float64, device=dev)
+        ws, wsb = _scan_workspace(B, L, dev)
+        call('asrn_clock_scan', ptr(x), ptr(y), B, L, 2 if reloj32 else 0, ptr(ws), wsb, stream_of(dev))
+        ctx.forma = (B, L, dev)
+        ctx.set_materialize_grads(False)
+        return y.view(B, L), y.view(B, L), la.view_as(la), la.view_as(la), x.view_as(x)
+
+    @staticmethod
+    def backward(ctx, g1, g2, l1, l2, add):
+        B, L, dev = ctx.forma
+        f64, f32 = torch.float64, torch.float32
+        gs = [None if g is None else _c(g, t) for g, t in ((g1, f64), (g2, f64), (add, f64), (l1, f32), (l2, f32))]
+        dbeta, dla = torch.empty((B, L), dtype=f64, device=dev), torch.empty((B, L), dtype=f32, device=dev)
+        ws, wsb = _scan_workspace(B, L, dev)
+        call('asrn_clock_bwd', *[ptr(g) for g in gs], B, L, ptr(dbeta), ptr(dla), ptr(ws), wsb, stream_of(dev))
+        return dbeta, dla, None
+
+
 # ---------------------------------------------------------------------------------------------------------------------
 # a12
 # ---------------------------------------------------------------------------------------------------------------------
@@ -567,10 +595,11 @@ class Streak(torch.autograd.Function):
 
 class Repeticion(torch.autograd.Function):
     """Hawkes and Streak in one pass (asrn_repetition_fwd/bwd: the B n Hawkes rows and the B streak rows share the
-    scans' launches): (hawkes (B, L, n), racha (B, L)), the same values and gradients as the two functions."""
+    scans' launches): (hawkes (B, L, n), racha (B, L)), the same values and gradients as the two functions. logs: kappa
+    and kappa_r are the rates' logarithms (the parameters), the exponentials and their gradients in the kernels."""
 
     @staticmethod
-    def forward(ctx, Bt, log_alfa, kappa, beta, kappa_r, order, rep, rank_k, vistos):
+    def forward(ctx, Bt, log_alfa, kappa, beta, kappa_r, order, rep, rank_k, vistos, logs=False):
         dev = _dev(Bt)
         B, n, L = order.shape
         Bt = _c(Bt, torch.float64)
@@ -587,8 +616,9 @@ class Repeticion(torch.autograd.Function):
             raise RuntimeError(f'repetition scans of {B * (n + 1)} rows x {L}: too many chunks')
         ws = torch.empty((wsb,), dtype=torch.uint8, device=dev) if wsb else None
         call('asrn_repetition_fwd', ptr(order), ptr(rep), ptr(Bt), ptr(la), ptr(kap), ptr(vistos), ptr(beta), ptr(kr),
-             B, L, n, ptr(hawkes), ptr(S), ptr(racha), ptr(ws), wsb, stream_of(dev))
+             int(logs), B, L, n, ptr(hawkes), ptr(S), ptr(racha), ptr(ws), wsb, stream_of(dev))
         ctx.save_for_backward(Bt, la, kap, order, rep, rank_k, S, vistos, beta, kr, racha)
+        ctx.logs = int(logs)
         return hawkes, racha
 
     @staticmethod
@@ -598,17 +628,20 @@ class Repeticion(torch.autograd.Function):
         dev = Bt.device
         gh = torch.zeros((B, L, n), dtype=torch.float32, device=dev) if gh is None else _c(gh, torch.float32)
         gr = torch.zeros((B, L), dtype=torch.float32, device=dev) if gr is None else _c(gr, torch.float32)
+        if B == 0 or L == 0:
+            return (torch.zeros_like(Bt), torch.zeros_like(la), torch.zeros_like(kap), torch.zeros_like(beta),
+                    torch.zeros_like(kr), None, None, None, None, None)
         dBt = torch.empty((B, L), dtype=torch.float64, device=dev)
         dla = torch.empty((B, L), dtype=torch.float32, device=dev)
-        dk = torch.empty((B, n), dtype=torch.float32, device=dev)
+        dk = torch.empty((n,), dtype=torch.float32, device=dev)
         dbeta = torch.empty((B, L), dtype=torch.float64, device=dev)
-        dkr = torch.empty((B,), dtype=torch.float32, device=dev)
+        dkr = torch.empty((1,), dtype=torch.float32, device=dev)
         wsb = query('asrn_repetition_bwd_workspace', B, L, n)
         ws = torch.empty((max(wsb, 1),), dtype=torch.uint8, device=dev)
         call('asrn_repetition_bwd', ptr(order), ptr(rep), ptr(rank_k), ptr(Bt), ptr(la), ptr(kap), ptr(S), ptr(gh),
-             ptr(vistos), ptr(beta), ptr(kr), ptr(racha), ptr(gr), B, L, n, ptr(dBt), ptr(dla), ptr(dk), ptr(dbeta),
-             ptr(dkr), ptr(ws), wsb, stream_of(dev))
-        return dBt, dla, dk.sum(0), dbeta, dkr.sum().reshape(1), None, None, None, None
+             ptr(vistos), ptr(beta), ptr(kr), ctx.logs, ptr(racha), ptr(gr), B, L, n, ptr(dBt), ptr(dla), ptr(dk),
+             ptr(dbeta), ptr(dkr), ptr(ws), wsb, stream_of(dev))
+        return dBt, dla, dk, dbeta, dkr, None, None, None, None, None
 
 
 # ---------------------------------------------------------------------------------------------------------------------

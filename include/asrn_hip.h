@@ -237,6 +237,10 @@ int asrn_copy_blocks(int32_t n, const float* const* src, float* const* dst, cons
  * workspace: asrn_scan_workspace(B, L) bytes. */
 int asrn_clock_scan(const double* x, double* y, int64_t B, int64_t L, int32_t mode, void* workspace,
                     int64_t workspace_bytes, void* stream);
+/* The clock's gradient and what joins it, in one pass: dbeta = suffix sums of (g1 + g2) + add, dlog_alfa = l1 + l2 (the
+ * gradients from the two users of the clock and of log alfa, and beta's other one; any may be null: zero). */
+int asrn_clock_bwd(const double* g1, const double* g2, const double* add, const float* l1, const float* l2, int64_t B,
+                   int64_t L, double* dbeta, float* dlog_alfa, void* workspace, int64_t workspace_bytes, void* stream);
 
 /* ---- a10: n-gram keys, stable key sort, repeated and seen flags -------------------------------------------------
  * Replaces _claves_de (asrn/nucleo.py:175-185), _ordenar_claves (asrn/nucleo.py:693-701) and the scatter of the seen
@@ -299,21 +303,22 @@ int asrn_streak_bwd(const float* vistos, const double* beta, const float* kappa_
 /* ---- a11: the repetition branch's two scans in shared launches (asrn/estable.py:304-321) -----------------------
  * asrn_hawkes_fwd and asrn_streak_fwd in one pass, the same outputs: the B n Hawkes rows and the B streak rows share
  * the scan's launches (the totals, the chunks and, backward, the per-row sums); asrn_repetition_bwd likewise stands
- * for asrn_hawkes_bwd and asrn_streak_bwd. Workspaces: asrn_repetition_workspace(B, L, n) bytes forward,
+ * for asrn_hawkes_bwd and asrn_streak_bwd, its dkappa (n) and dkappa_r (1) summed over the batch rows in order. logs:
+ * kappa and kappa_r hold the rates' logarithms, and their gradients are those of the logarithms. Workspaces: asrn_repetition_workspace(B, L, n) bytes forward,
  * asrn_repetition_bwd_workspace(B, L, n) backward. No reference counterpart as one call: the reference runs the two
  * scans one after the other in _repeticion. */
 int64_t asrn_repetition_workspace(int64_t B, int64_t L, int32_t n);
 int asrn_repetition_fwd(const int32_t* order, const uint8_t* repeated, const double* Bt, const float* log_alfa,
-                        const float* kappa, const float* vistos, const double* beta, const float* kappa_r, int64_t B,
-                        int64_t L, int32_t n, float* hawkes, float* S_sorted, float* racha, void* workspace,
-                        int64_t workspace_bytes, void* stream);
+                        const float* kappa, const float* vistos, const double* beta, const float* kappa_r,
+                        int32_t logs, int64_t B, int64_t L, int32_t n, float* hawkes, float* S_sorted, float* racha,
+                        void* workspace, int64_t workspace_bytes, void* stream);
 int64_t asrn_repetition_bwd_workspace(int64_t B, int64_t L, int32_t n);
 int asrn_repetition_bwd(const int32_t* order, const uint8_t* repeated, const int32_t* rank_k, const double* Bt,
                         const float* log_alfa, const float* kappa, const float* S_sorted, const float* dhawkes,
-                        const float* vistos, const double* beta, const float* kappa_r, const float* racha,
-                        const float* dracha, int64_t B, int64_t L, int32_t n, double* dBt, float* dlog_alfa,
-                        float* dkappa, double* dbeta, float* dkappa_r, void* workspace, int64_t workspace_bytes,
-                        void* stream);
+                        const float* vistos, const double* beta, const float* kappa_r, int32_t logs,
+                        const float* racha, const float* dracha, int64_t B, int64_t L, int32_t n, double* dBt,
+                        float* dlog_alfa, float* dkappa, double* dbeta, float* dkappa_r, void* workspace,
+                        int64_t workspace_bytes, void* stream);
 
 /* ---- a13: the gate consumer (asrn/estable.py:376-403, asrn/nucleo.py:865-878) -------------------------------
  * Replaces the PyTorch ops of _combinar after W_o: with A = W_o salida (B*L, d) (fp32, or bf16 when aporte_bf16),
