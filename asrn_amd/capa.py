@@ -368,15 +368,16 @@ class CapaASRNEstable(nn.Module):
 
     # --- all together -----------------------------------------------------------------------------------------------
 
-    def forward(self, E, h, piezas=None, ngramas=None):
+    def forward(self, E, h, piezas=None, ngramas=None, una_corriente=False):
         """E (B, L, d), h (B, L, d), piezas (B, L) or None -> h' (B, L, d) (asrn/estable.py:407-421).
 
         ngramas: what `ngramas(piezas, capa)` returned for these token ids, to share one n-gram sort between every ASRN
         layer of a model (it depends on the tokens only; the reference sorts again in each layer, nucleo:688-701).
-        Without it the layer sorts itself."""
-        return self._adelante(E, h, piezas, ngramas=ngramas)
+        Without it the layer sorts itself. una_corriente: both branches on the current stream (ModeloASRN's small
+        batches)."""
+        return self._adelante(E, h, piezas, ngramas=ngramas, una_corriente=una_corriente)
 
-    def _adelante(self, E, h, piezas=None, partes=None, ngramas=None):
+    def _adelante(self, E, h, piezas=None, partes=None, ngramas=None, una_corriente=False):
         """forward; with a dict `partes`, also keeps what the generation step starts from (the prompt's phi, V,
         Qc, Kc, sig, beta, Bt, log_alfa, n-gram keys and their sort, hawkes and racha)."""
         self._revisar(E)
@@ -390,7 +391,8 @@ class CapaASRNEstable(nn.Module):
         # one, beside the hash producers and the bucket sort; the candidate attention waits for the context only.
         # Autograd runs each op's backward on the stream of its forward, so the backward overlaps the same way, and
         # the W_o W_v projection's weight gradient (_Gemelo) runs there too.
-        principal, lado = torch.cuda.current_stream(E.device), _lateral(E.device)
+        principal = torch.cuda.current_stream(E.device)
+        lado = principal if una_corriente else _lateral(E.device)
         pesos = self._pesos(E)
         lado.wait_stream(principal)
         with torch.cuda.stream(lado):

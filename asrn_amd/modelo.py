@@ -24,6 +24,11 @@ MEZCLAS = ('conv', 'memoria')
 OPCIONES_CAPA = ('n_tablas', 'n_bits', 'afin_oculto', 'chunk', 'tablas_contexto', 'confirmar', 'sufijo', 'vistos',
                  'nodos_racha', 'racha_max')
 MODOS_CHECKPOINT = ('no', 'asrn', 'todo')
+# Embedding values (B L d) up to which a model's training step keeps its ASRN layers on one stream: a captured step
+# without branches replays with its launches back to back, one with a branch pays for them one by one, and below this
+# the launches cost more than the layers' two branches gain by running side by side (us a step, two streams / one: 512
+# tokens at d 64 690 / 599, 4096 at d 64 785 / 723, 4096 at d 256 1365 / 1324, 4096 at d 512 2588 / 2603)
+UNA_CORRIENTE = 1 << 20
 
 
 def _base(modelo):
@@ -200,6 +205,7 @@ class ModeloASRN(nn.Module):
         ck_capa = recalcular and self.checkpoint != 'no'
         # the n-gram sort depends on the token ids only: one for every ASRN layer
         ng = ngramas(x, self.largos[0]) if len(self.largos) and x.is_cuda else None
+        una = recalcular and E.numel() <= UNA_CORRIENTE and ops.incrustar_ok(self.emb, x)
         capas = iter(self.largos)
         h = E
         for i, bloque in enumerate(self.bloques):
@@ -207,9 +213,10 @@ class ModeloASRN(nn.Module):
             if i in self.pos_largo:
                 capa = next(capas)
                 if ck_capa:
-                    h = torch.utils.checkpoint.checkpoint(capa, E, h, x, use_reentrant=False, ngramas=ng)
+                    h = torch.utils.checkpoint.checkpoint(capa, E, h, x, use_reentrant=False, ngramas=ng,
+                                                          una_corriente=una)
                 else:
-                    h = capa(E, h, x, ngramas=ng)
+                    h = capa(E, h, x, ngramas=ng, una_corriente=una)
         return h
 
     def forward(self, x):

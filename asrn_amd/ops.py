@@ -1358,16 +1358,19 @@ class Incrustar(torch.autograd.Function):
         return dw, None
 
 
-def incrustar(emb, x):
-    """emb(x); for a plain fp32 nn.Embedding in training on up to FICHAS_INCRUSTAR int64 tokens, with asrn_embedding_bwd
-    as its backward."""
+def incrustar_ok(emb, x):
+    """Whether incrustar(emb, x) runs asrn_embedding_bwd: a plain fp32 nn.Embedding in training on the GPU, up to
+    FICHAS_INCRUSTAR int64 tokens."""
     w = emb.weight
-    if (w.is_cuda and x.device == w.device and x.dtype == torch.int64 and w.dtype == torch.float32 and w.requires_grad
+    return (w.is_cuda and x.device == w.device and x.dtype == torch.int64 and w.dtype == torch.float32 and w.requires_grad
             and torch.is_grad_enabled() and 1 <= x.numel() <= FICHAS_INCRUSTAR and type(emb) is torch.nn.Embedding
             and emb.padding_idx is None and emb.max_norm is None and not emb.scale_grad_by_freq and not emb.sparse
-            and not emb._forward_hooks and not emb._forward_pre_hooks and not emb._backward_hooks):
-        return Incrustar.apply(w, x)
-    return emb(x)
+            and not emb._forward_hooks and not emb._forward_pre_hooks and not emb._backward_hooks)
+
+
+def incrustar(emb, x):
+    """emb(x), with asrn_embedding_bwd as its backward where incrustar_ok."""
+    return Incrustar.apply(emb.weight, x) if incrustar_ok(emb, x) else emb(x)
 
 
 # ---------------------------------------------------------------------------------------------------------------------
