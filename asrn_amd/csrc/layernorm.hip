@@ -5,6 +5,10 @@
 //   backward  from dy (fp32 or bf16): g = dy gamma, dx = rstd (g - mean(g) - xhat mean(g xhat)) [+ dres, the gradient
 //             of the same x through the residual path, so that autograd adds nothing], and d gamma = sum dy xhat,
 //             d beta = sum dy as per-workgroup partial rows summed in a fixed order by asrn_column_sums.
+// The local block's middle is fused into its second LayerNorm (GC: c, the convolution's output, in fp32 or bf16): forward
+// x = h + gelu(c), kept for the residual path, then the norm of x; backward also dc = gelu'(c) dx, each rounded where
+// autocast's separate ops round (gelu's output, dx and dc to c's dtype). HBM-bound; at 16,384 rows of 768 in bf16 the
+// forward's three kernels took 52 us and the backward's three 68 us, the fused ones 29 and 46.
 // Forward: a workgroup takes 8 rows, each wave 2 with both rows (float4 per lane) loaded at once. Backward: a workgroup
 // takes 32 rows, each wave 8 of them, 2 rows' loads at a time.
 #include "common.h"
@@ -25,7 +29,14 @@ struct LnArgs {
   int64_t rows; int d; float eps;
   void* y; int64_t ldy; float2* stats;                                   // forward
   const void* dy; int64_t lddy; const float* dres; float* dx; float* partial;   // backward (dx and dres: ldx)
+  const void* c; float* xout; void* dc;     // GC: c (rows, d) dense; forward x + gelu(c) out (ldx); backward dc out
 };
+
+// exact GELU and its derivative, as torch forms them in fp32
+__device__ __forceinline__ float ln_gelu(float x) { return x * 0.5f * (1.f + erff(x * 0.70710678118654752f)); }
+__device__ __forceinline__ float ln_dgelu(float x) {
+  return 0.5f * (1.f + erff(x * 0.70710678118654752f)) + x * (expf(-0.5f * x * x) * 0.39894228040143268f);
+}
 
 __device__ __forceinline__ uint32_t ln_bf16(float v) {
   const uint32_t u = __float_as_uint(v);
@@ -40,9 +51,16 @@ __device__ __forceinline__ float4 ld_row4(const void* p, bool b16, int64_t off4)
   }
   return reinterpret_cast<const float4*>(p)[off4];
 }
+// v rounded to bf16 and back
+__device__ __forceinline__ float ln_round(float v) { return __uint_as_float(ln_bf16(v) << 16); }
+template <bool B16, class F>
+__device__ __forceinline__ float4 ln_map(float4 v, F f) {
+  const float4 r = make_float4(f(v.x), f(v.y), f(v.z), f(v.w));
+  return B16 ? make_float4(ln_round(r.x), ln_round(r.y), ln_round(r.z), ln_round(r.w)) : r;
+}
 __device__ __forceinline__ float ln_dot4(float4 a, float4 b) { return a.x * b.x + a.y * b.y + a.z * b.z + a.w * b.w; }
 
-template <int D4, bool OB16>
+template <int D4, bool OB16, int GC>
 __global__ __launch_bounds__(kLnThreads) void k_ln_fwd(LnArgs a) {
   const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x >> 6;
   const int d4 = a.d >> 2;
@@ -60,6 +78,11 @@ __global__ __launch_bounds__(kLnThreads) void k_ln_fwd(LnArgs a) {
       xv[u][k] = make_float4(0.f, 0.f, 0.f, 0.f);
       if (r < a.rows && q < d4) {
         xv[u][k] = reinterpret_cast<const float4*>(a.x + r * a.ldx)[q];
+        if constexpr (GC > 0) {
+          const float4 g = ln_map<GC == 2>(ld_row4(a.c, GC == 2, r * d4 + q), ln_gelu);
+          xv[u][k].x += g.x; xv[u][k].y += g.y; xv[u][k].z += g.z; xv[u][k].w += g.w;
+          reinterpret_cast<float4*>(a.xout + r * a.ldx)[q] = xv[u][k];
+        }
         s[u] += (xv[u][k].x + xv[u][k].y) + (xv[u][k].z + xv[u][k].w);
       }
     }
@@ -98,7 +121,7 @@ __global__ __launch_bounds__(kLnThreads) void k_ln_fwd(LnArgs a) {
   }
 }
 
-template <int D4, bool DB16>
+template <int D4, bool DB16, int GC>
 __global__ __launch_bounds__(kLnThreads) void k_ln_bwd(LnArgs a) {
   __shared__ float red[kLnWaves][2 * 4 * D4 * kWave];
   const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x >> 6;
@@ -109,7 +132,7 @@ __global__ __launch_bounds__(kLnThreads) void k_ln_bwd(LnArgs a) {
 #pragma unroll
   for (int k = 0; k < D4; ++k) gw[k] = gb[k] = make_float4(0.f, 0.f, 0.f, 0.f);
   for (int b = 0; b < kLnBwdPerWave; b += kLnBatch) {
-    float4 xv[kLnBatch][D4], dv[kLnBatch][D4], rv[kLnBatch][D4];
+    float4 xv[kLnBatch][D4], dv[kLnBatch][D4], rv[kLnBatch][D4], cv[kLnBatch][GC > 0 ? D4 : 1];
     float2 st[kLnBatch];
 #pragma unroll
     for (int u = 0; u < kLnBatch; ++u) {
@@ -125,6 +148,7 @@ __global__ __launch_bounds__(kLnThreads) void k_ln_bwd(LnArgs a) {
           dv[u][k] = DB16 ? ld_row4(reinterpret_cast<const uint16_t*>(a.dy) + r * a.lddy, true, q)
                           : ld_row4(reinterpret_cast<const float*>(a.dy) + r * a.lddy, false, q);
           if (a.dres) rv[u][k] = reinterpret_cast<const float4*>(a.dres + r * a.ldx)[q];
+          if constexpr (GC > 0) cv[u][k] = ld_row4(a.c, GC == 2, r * d4 + q);
         }
       }
     }
@@ -155,10 +179,21 @@ __global__ __launch_bounds__(kLnThreads) void k_ln_bwd(LnArgs a) {
 #pragma unroll
       for (int k = 0; k < D4; ++k) {
         const int q = lane + kWave * k;
-        if (q < d4)
-          reinterpret_cast<float4*>(a.dx + r * a.ldx)[q] =
+        if (q < d4) {
+          const float4 dx =
               make_float4(rstd * (g[k].x - m1 - xh[k].x * m2) + rv[u][k].x, rstd * (g[k].y - m1 - xh[k].y * m2) + rv[u][k].y,
                           rstd * (g[k].z - m1 - xh[k].z * m2) + rv[u][k].z, rstd * (g[k].w - m1 - xh[k].w * m2) + rv[u][k].w);
+          reinterpret_cast<float4*>(a.dx + r * a.ldx)[q] = dx;
+          if constexpr (GC > 0) {
+            const float4 e = ln_map<GC == 2>(dx, [](float v) { return v; }), w = ln_map<false>(cv[u][k], ln_dgelu);
+            const float4 dc = make_float4(e.x * w.x, e.y * w.y, e.z * w.z, e.w * w.w);
+            if constexpr (GC == 2)
+              reinterpret_cast<uint2*>(a.dc)[r * d4 + q] =
+                  make_uint2(ln_bf16(dc.x) | (ln_bf16(dc.y) << 16), ln_bf16(dc.z) | (ln_bf16(dc.w) << 16));
+            else
+              reinterpret_cast<float4*>(a.dc)[r * d4 + q] = dc;
+          }
+        }
       }
     }
   }
@@ -190,33 +225,83 @@ static int ln_d4(int d) { return (d + 4 * kWave - 1) / (4 * kWave); }
 
 using namespace asrn;
 
+// GC of c: 0 none, 1 fp32, 2 bf16
+#define LN_GC(KERNEL, D4, B16)                                                                        \
+  if (gc == 0) hipLaunchKernelGGL((KERNEL<D4, B16, 0>), grid, block, 0, st, a);                       \
+  else if (gc == 1) hipLaunchKernelGGL((KERNEL<D4, B16, 1>), grid, block, 0, st, a);                  \
+  else hipLaunchKernelGGL((KERNEL<D4, B16, 2>), grid, block, 0, st, a);
+#define LN_B16(KERNEL, D4) \
+  if (b16) { LN_GC(KERNEL, D4, true) } else { LN_GC(KERNEL, D4, false) }
+#define LN_LAUNCH(KERNEL)                  \
+  switch (ln_d4(a.d)) {                    \
+    case 1: LN_B16(KERNEL, 1) break;       \
+    case 2: LN_B16(KERNEL, 2) break;       \
+    case 3: LN_B16(KERNEL, 3) break;       \
+    default: LN_B16(KERNEL, 4) break;      \
+  }
+
+static int ln_fwd(LnArgs a, bool b16, int gc, hipStream_t st, const char* what) {
+  ASRN_REQUIRE(a.rows >= 0 && a.d > 0 && a.d % 4 == 0 && a.d <= 4 * kLnMaxD4 * kWave && a.ldx >= a.d &&
+                   a.ldx % 4 == 0 && a.ldy >= a.d && a.ldy % 4 == 0 && a.eps > 0.f,
+               "%s: bad sizes rows=%lld d=%d (a multiple of 4, <= %d) ldx=%lld ldy=%lld", what, (long long)a.rows, a.d,
+               4 * kLnMaxD4 * kWave, (long long)a.ldx, (long long)a.ldy);
+  if (a.rows == 0) return 0;
+  ASRN_REQUIRE(((uintptr_t)a.x & 15) == 0 && ((uintptr_t)a.y & (b16 ? 7 : 15)) == 0 && ((uintptr_t)a.gamma & 15) == 0 &&
+                   ((uintptr_t)a.beta & 15) == 0 && ((uintptr_t)a.c & (gc == 2 ? 7 : 15)) == 0 &&
+                   ((uintptr_t)a.xout & 15) == 0,
+               "%s: rows and parameters must be 16-byte aligned (8 for bf16)", what);
+  const dim3 grid((unsigned)((a.rows + kLnFwdRows - 1) / kLnFwdRows)), block(kLnThreads);
+  LN_LAUNCH(k_ln_fwd)
+  return check_launch(what);
+}
+
+static int ln_bwd(LnArgs a, bool b16, int gc, float* dparams, void* workspace, int64_t workspace_bytes, void* stream,
+                  const char* what) {
+  ASRN_REQUIRE(a.rows >= 0 && a.d > 0 && a.d % 4 == 0 && a.d <= 4 * kLnMaxD4 * kWave && a.ldx >= a.d &&
+                   a.ldx % 4 == 0 && a.lddy >= a.d && a.lddy % 4 == 0,
+               "%s: bad sizes rows=%lld d=%d (a multiple of 4, <= %d) ldx=%lld lddy=%lld", what, (long long)a.rows,
+               a.d, 4 * kLnMaxD4 * kWave, (long long)a.ldx, (long long)a.lddy);
+  const int64_t need = asrn_layer_norm_bwd_workspace(a.rows, a.d);
+  ASRN_REQUIRE(need >= 0 && workspace_bytes >= need && workspace != nullptr && ((uintptr_t)workspace % 256) == 0,
+               "%s: needs a 256-byte aligned workspace of %lld bytes", what, (long long)need);
+  if (a.rows == 0)
+    return asrn_column_sums(nullptr, 0, 0, 2 * (int64_t)a.d, 2 * (int64_t)a.d, dparams, nullptr, 0, stream);
+  ASRN_REQUIRE(((uintptr_t)a.x & 15) == 0 && ((uintptr_t)a.dx & 15) == 0 && ((uintptr_t)a.dy & (b16 ? 7 : 15)) == 0 &&
+                   ((uintptr_t)a.dres & 15) == 0 && ((uintptr_t)a.gamma & 15) == 0 &&
+                   (((uintptr_t)a.c | (uintptr_t)a.dc) & (gc == 2 ? 7 : 15)) == 0,
+               "%s: rows and parameters must be 16-byte aligned (8 for bf16)", what);
+  a.partial = (float*)workspace;
+  const int64_t groups = ln_bwd_groups(a.rows);
+  ASRN_REQUIRE(groups < (int64_t(1) << 31), "%s: too many rows", what);
+  const dim3 grid((unsigned)groups), block(kLnThreads);
+  hipStream_t st = (hipStream_t)stream;
+  LN_LAUNCH(k_ln_bwd)
+  if (check_launch(what)) return 1;
+  // one launch for up to 1,024 partial rows (two rounds of its loads); more are summed in two levels
+  if (groups <= 1024) return group_sums(a.partial, (int)groups, 2 * a.d, dparams, st);
+  const int64_t part_bytes = (groups * 2 * a.d * 4 + 255) / 256 * 256;
+  return asrn_column_sums(a.partial, 0, groups, 2 * (int64_t)a.d, 2 * (int64_t)a.d, dparams,
+                          (char*)workspace + part_bytes, need - part_bytes, stream);
+}
+
 extern "C" int asrn_layer_norm_fwd(const float* x, int64_t ldx, const float* gamma, const float* beta, int64_t rows,
                                    int32_t d, float eps, int32_t out_bf16, void* y, int64_t ldy, float* stats,
                                    void* stream) {
-  ASRN_REQUIRE(rows >= 0 && d > 0 && d % 4 == 0 && d <= 4 * kLnMaxD4 * kWave && ldx >= d && ldx % 4 == 0 &&
-                   ldy >= d && ldy % 4 == 0 && eps > 0.f && (out_bf16 == 0 || out_bf16 == 1),
-               "asrn_layer_norm_fwd: bad sizes rows=%lld d=%d (a multiple of 4, <= %d) ldx=%lld ldy=%lld",
-               (long long)rows, d, 4 * kLnMaxD4 * kWave, (long long)ldx, (long long)ldy);
-  if (rows == 0) return 0;
-  ASRN_REQUIRE(((uintptr_t)x & 15) == 0 && ((uintptr_t)y & (out_bf16 ? 7 : 15)) == 0 && ((uintptr_t)gamma & 15) == 0 &&
-                   ((uintptr_t)beta & 15) == 0,
-               "asrn_layer_norm_fwd: rows and parameters must be 16-byte aligned (8 for bf16 output)");
   LnArgs a{};
   a.x = x; a.ldx = ldx; a.gamma = gamma; a.beta = beta; a.rows = rows; a.d = d; a.eps = eps; a.y = y; a.ldy = ldy;
   a.stats = reinterpret_cast<float2*>(stats);
-  const dim3 grid((unsigned)((rows + kLnFwdRows - 1) / kLnFwdRows)), block(kLnThreads);
-  hipStream_t st = (hipStream_t)stream;
-#define LN_FWD(D4)                                                                                   \
-  if (out_bf16) hipLaunchKernelGGL((k_ln_fwd<D4, true>), grid, block, 0, st, a);                    \
-  else hipLaunchKernelGGL((k_ln_fwd<D4, false>), grid, block, 0, st, a);
-  switch (ln_d4(d)) {
-    case 1: LN_FWD(1) break;
-    case 2: LN_FWD(2) break;
-    case 3: LN_FWD(3) break;
-    default: LN_FWD(4) break;
-  }
-#undef LN_FWD
-  return check_launch("asrn_layer_norm_fwd");
+  ASRN_REQUIRE(out_bf16 == 0 || out_bf16 == 1, "asrn_layer_norm_fwd: out_bf16 must be 0 or 1");
+  return ln_fwd(a, out_bf16, 0, (hipStream_t)stream, "asrn_layer_norm_fwd");
+}
+
+extern "C" int asrn_gelu_norm_fwd(const float* h, const void* c, int32_t c_bf16, const float* gamma, const float* beta,
+                                  int64_t rows, int32_t d, float eps, int32_t out_bf16, float* x, void* y,
+                                  float* stats, void* stream) {
+  LnArgs a{};
+  a.x = h; a.ldx = d; a.gamma = gamma; a.beta = beta; a.rows = rows; a.d = d; a.eps = eps; a.y = y; a.ldy = d;
+  a.stats = reinterpret_cast<float2*>(stats); a.c = c; a.xout = x;
+  ASRN_REQUIRE(rows == 0 || (c && x), "asrn_gelu_norm_fwd: null c or x");
+  return ln_fwd(a, out_bf16 != 0, c_bf16 ? 2 : 1, (hipStream_t)stream, "asrn_gelu_norm_fwd");
 }
 
 extern "C" int64_t asrn_layer_norm_bwd_workspace(int64_t rows, int32_t d) {
@@ -231,36 +316,20 @@ extern "C" int asrn_layer_norm_bwd(const float* x, int64_t ldx, const float* gam
                                    int32_t d, const void* dy, int32_t dy_bf16, int64_t lddy, const float* dres,
                                    float* dx, float* dparams, void* workspace, int64_t workspace_bytes,
                                    void* stream) {
-  ASRN_REQUIRE(rows >= 0 && d > 0 && d % 4 == 0 && d <= 4 * kLnMaxD4 * kWave && ldx >= d && ldx % 4 == 0 &&
-                   lddy >= d && lddy % 4 == 0 && (dy_bf16 == 0 || dy_bf16 == 1),
-               "asrn_layer_norm_bwd: bad sizes rows=%lld d=%d (a multiple of 4, <= %d) ldx=%lld lddy=%lld",
-               (long long)rows, d, 4 * kLnMaxD4 * kWave, (long long)ldx, (long long)lddy);
-  const int64_t need = asrn_layer_norm_bwd_workspace(rows, d);
-  ASRN_REQUIRE(need >= 0 && workspace_bytes >= need && workspace != nullptr && ((uintptr_t)workspace % 256) == 0,
-               "asrn_layer_norm_bwd: needs a 256-byte aligned workspace of %lld bytes", (long long)need);
-  if (rows == 0) return asrn_column_sums(nullptr, 0, 0, 2 * (int64_t)d, 2 * (int64_t)d, dparams, nullptr, 0, stream);
-  ASRN_REQUIRE(((uintptr_t)x & 15) == 0 && ((uintptr_t)dx & 15) == 0 && ((uintptr_t)dy & (dy_bf16 ? 7 : 15)) == 0 &&
-                   ((uintptr_t)dres & 15) == 0 && ((uintptr_t)gamma & 15) == 0,
-               "asrn_layer_norm_bwd: rows and parameters must be 16-byte aligned (8 for bf16 dy)");
   LnArgs a{};
   a.x = x; a.ldx = ldx; a.gamma = gamma; a.rows = rows; a.d = d; a.stats = reinterpret_cast<float2*>(const_cast<float*>(stats));
-  a.dy = dy; a.lddy = lddy; a.dres = dres; a.dx = dx; a.partial = (float*)workspace;
-  const int64_t groups = ln_bwd_groups(rows);
-  ASRN_REQUIRE(groups < (int64_t(1) << 31), "asrn_layer_norm_bwd: too many rows");
-  const dim3 grid((unsigned)groups), block(kLnThreads);
-  hipStream_t st = (hipStream_t)stream;
-#define LN_BWD(D4)                                                                                   \
-  if (dy_bf16) hipLaunchKernelGGL((k_ln_bwd<D4, true>), grid, block, 0, st, a);                     \
-  else hipLaunchKernelGGL((k_ln_bwd<D4, false>), grid, block, 0, st, a);
-  switch (ln_d4(d)) {
-    case 1: LN_BWD(1) break;
-    case 2: LN_BWD(2) break;
-    case 3: LN_BWD(3) break;
-    default: LN_BWD(4) break;
-  }
-#undef LN_BWD
-  if (check_launch("asrn_layer_norm_bwd")) return 1;
-  const int64_t part_bytes = (groups * 2 * d * 4 + 255) / 256 * 256;
-  return asrn_column_sums(a.partial, 0, groups, 2 * (int64_t)d, 2 * (int64_t)d, dparams,
-                          (char*)workspace + part_bytes, need - part_bytes, stream);
+  a.dy = dy; a.lddy = lddy; a.dres = dres; a.dx = dx;
+  ASRN_REQUIRE(dy_bf16 == 0 || dy_bf16 == 1, "asrn_layer_norm_bwd: dy_bf16 must be 0 or 1");
+  return ln_bwd(a, dy_bf16, 0, dparams, workspace, workspace_bytes, stream, "asrn_layer_norm_bwd");
+}
+
+extern "C" int asrn_gelu_norm_bwd(const float* x, const void* c, int32_t c_bf16, const float* gamma, const float* stats,
+                                  int64_t rows, int32_t d, const void* dy, int32_t dy_bf16, const float* dres,
+                                  float* dx, void* dc, float* dparams, void* workspace, int64_t workspace_bytes,
+                                  void* stream) {
+  LnArgs a{};
+  a.x = x; a.ldx = d; a.gamma = gamma; a.rows = rows; a.d = d; a.stats = reinterpret_cast<float2*>(const_cast<float*>(stats));
+  a.dy = dy; a.lddy = d; a.dres = dres; a.dx = dx; a.c = c; a.dc = dc;
+  ASRN_REQUIRE(rows == 0 || (c && dc), "asrn_gelu_norm_bwd: null c or dc");
+  return ln_bwd(a, dy_bf16 != 0, c_bf16 ? 2 : 1, dparams, workspace, workspace_bytes, stream, "asrn_gelu_norm_bwd");
 }

@@ -123,6 +123,9 @@ class BloqueLocal(nn.Module):
             c = conv_causal(z, self.conv.weight, self.conv.bias)
         else:
             c = conv_canal_causal(z, self.conv.weight, self.conv.bias)
+        if self.mezcla == 'conv' and not (self.drop.training and self.drop.p > 0):
+            y, h = ops.suma_gelu_norma(self.ln2, h, c, _dtype_producto(h))
+            return h + self._ff(y)
         c = F.gelu(c)
         if self.mezcla == 'memoria':
             c = c + self._memoria(z)

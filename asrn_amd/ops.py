@@ -1476,6 +1476,56 @@ class NormaResidual(torch.autograd.Function):
         return dx.view(*lead, d).to(xdt), dp[:d].view(gshape), dp[d:].view(bshape), None, None
 
 
+class SumaGeluNorma(torch.autograd.Function):
+    """The middle of a 'conv' local block (asrn/nucleo.py:969-1014): x = h + gelu(c) with c the convolution's output, and
+    the LayerNorm of x, in one kernel each way (asrn_gelu_norm_fwd/bwd): returns (the norm in `dtype`, x). h fp32, c fp32
+    or bf16 of the same shape; every value rounds where the separate ops round."""
+
+    @staticmethod
+    def forward(ctx, h, c, gamma, beta, eps, dtype):
+        dev = _dev(h)
+        d, lead = h.shape[-1], h.shape[:-1]
+        h2, c2 = h.contiguous().reshape(-1, d), c.contiguous().reshape(-1, d)
+        rows = h2.shape[0]
+        g, b = _c(gamma, torch.float32), _c(beta, torch.float32)
+        x = torch.empty((rows, d), dtype=torch.float32, device=dev)
+        y = torch.empty((rows, d), dtype=dtype, device=dev)
+        stats = torch.empty((rows, 2), dtype=torch.float32, device=dev)
+        call('asrn_gelu_norm_fwd', ptr(h2), ptr(c2), int(c2.dtype == torch.bfloat16), ptr(g), ptr(b), rows, d, float(eps),
+             int(dtype == torch.bfloat16), ptr(x), ptr(y), ptr(stats), stream_of(dev))
+        ctx.save_for_backward(x, c2, g, stats)
+        ctx.meta = (lead, gamma.shape, beta.shape)
+        return y.view(*lead, d), x.view(*lead, d)
+
+    @staticmethod
+    def backward(ctx, dy, dres):
+        x, c2, g, stats = ctx.saved_tensors
+        lead, gshape, bshape = ctx.meta
+        rows, d = x.shape
+        dev = x.device
+        bf16 = dy.dtype == torch.bfloat16
+        dyc = (_c(dy) if bf16 else _c(dy, torch.float32)).reshape(rows, d)
+        dr = None if dres is None else _c(dres, torch.float32).reshape(rows, d)
+        dx, dc = torch.empty_like(x), torch.empty_like(c2)
+        dp = torch.empty((2 * d,), dtype=torch.float32, device=dev)
+        wsb = query('asrn_layer_norm_bwd_workspace', rows, d)
+        ws = torch.empty((wsb,), dtype=torch.uint8, device=dev)
+        call('asrn_gelu_norm_bwd', ptr(x), ptr(c2), int(c2.dtype == torch.bfloat16), ptr(g), ptr(stats), rows, d, ptr(dyc),
+             int(bf16), ptr(dr), ptr(dx), ptr(dc), ptr(dp), ptr(ws), wsb, stream_of(dev))
+        return dx.view(*lead, d), dc.view(*lead, d), dp[:d].view(gshape), dp[d:].view(bshape), None, None
+
+
+def suma_gelu_norma(ln, h, c, dtype):
+    """(LayerNorm ln of h + gelu(c) in `dtype`, h + gelu(c)): fused where norma_residual's is and h is fp32, c fp32 or
+    bf16; else the separate ops."""
+    d = h.shape[-1]
+    if (h.is_cuda and h.dtype == torch.float32 and c.dtype in (torch.float32, torch.bfloat16) and c.shape == h.shape
+            and dtype in (torch.float32, torch.bfloat16) and d % 4 == 0 and d <= 1024 and ln.elementwise_affine
+            and ln.bias is not None and tuple(ln.normalized_shape) == (d,)):
+        return SumaGeluNorma.apply(h, c, ln.weight, ln.bias, ln.eps, dtype)
+    return norma_residual(ln, h + F.gelu(c), dtype)
+
+
 def norma_residual(ln, x, dtype):
     """(LayerNorm ln of x in `dtype`, x for the residual path): the library's fused LayerNorm for fp32 x on the GPU
     with d a multiple of 4 up to 1024, else ln(x) (cast to dtype) and x itself."""

@@ -620,6 +620,15 @@ int64_t asrn_layer_norm_bwd_workspace(int64_t rows, int32_t d);
 int asrn_layer_norm_bwd(const float* x, int64_t ldx, const float* gamma, const float* stats, int64_t rows, int32_t d,
                         const void* dy, int32_t dy_bf16, int64_t lddy, const float* dres, float* dx, float* dparams,
                         void* workspace, int64_t workspace_bytes, void* stream);
+/* The same with a local block's middle in it (asrn/nucleo.py:969-1014): x (rows, d) = h + gelu(c), c (rows, d) fp32 or
+ * bf16 (gelu's result rounded to c's dtype before the sum, as the separate ops round), y the norm of x; backward dx as
+ * above and dc = gelu'(c) dx in c's dtype (dx rounded to it first). Dense rows. */
+int asrn_gelu_norm_fwd(const float* h, const void* c, int32_t c_bf16, const float* gamma, const float* beta,
+                       int64_t rows, int32_t d, float eps, int32_t out_bf16, float* x, void* y, float* stats,
+                       void* stream);
+int asrn_gelu_norm_bwd(const float* x, const void* c, int32_t c_bf16, const float* gamma, const float* stats,
+                       int64_t rows, int32_t d, const void* dy, int32_t dy_bf16, const float* dres, float* dx, void* dc,
+                       float* dparams, void* workspace, int64_t workspace_bytes, void* stream);
 
 #ifdef __cplusplus
 }
