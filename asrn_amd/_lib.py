@@ -87,6 +87,8 @@ SIGNATURES = {
     'asrn_embedding_bwd': (ctypes.c_int, [_P, _P, _I64, _I64, _I32, _P, _P]),
     'asrn_clip_gradients_workspace': (_I64, [_I32, _P]),
     'asrn_clip_gradients': (ctypes.c_int, [_I32, _P, _P, _F32, _P, _P, _P, _P, _I64, _P]),
+    'asrn_key_rows_fwd': (ctypes.c_int, [_P, _I64, _I64, _I32, _P, _P, _P]),
+    'asrn_key_rows_bwd': (ctypes.c_int, [_P, _P, _P, _I64, _I64, _I32, _P, _P]),
     'asrn_conv_window_fwd': (ctypes.c_int, [_P, _I64, _I64, _I64, _I32, _I32, _I32, _P, _P]),
     'asrn_conv_window_bwd': (ctypes.c_int, [_P, _I32, _I64, _I64, _I32, _I32, _P, _I64, _P]),
     'asrn_layer_norm_fwd': (ctypes.c_int, [_P, _I64, _P, _P, _I64, _I32, _F32, _I32, _P, _I64, _P, _P]),

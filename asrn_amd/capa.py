@@ -185,11 +185,13 @@ class CapaASRNEstable(nn.Module):
             # MLP's on the key [E_t; E_{t-1}] built from the 16-bit E, each rounded once. Split by linearity, the
             # context layer would round W_a E_t and W_b E_{t-1} apart: one 16-bit rounding more, which moves phi
             # values near 0 to the other sign and their positions to other buckets than the reference's
-            E16 = _a_autocast(E)
-            llave = torch.cat([E16, F.pad(E16, (0, 0, 1, 0))[:, :E16.shape[1]]], dim=-1)
+            if torch.get_autocast_dtype(E.device.type) == torch.bfloat16 and ops.claves16_ok(E):
+                E16, filas, llave = ops.Claves16.apply(E)
+            else:
+                E16 = filas = _a_autocast(E)
+                llave = torch.cat([E16, F.pad(E16, (0, 0, 1, 0))[:, :E16.shape[1]]], dim=-1)
             g = F.gelu(torch.cat([lineal(E16, pal[0].weight, pal[0].bias), lineal(llave, ctx[0].weight, ctx[0].bias)],
                                  dim=-1))
-            filas = E16
         else:
             y = lineal(E, W, F.pad(pal[0].bias, (0, 2 * mc)), propio=False)
             hp, za, zb = y.split([m, mc, mc], dim=-1)

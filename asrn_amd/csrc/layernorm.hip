@@ -8,7 +8,7 @@
 // The local block's middle is fused into its second LayerNorm (GC: c, the convolution's output, in fp32 or bf16): forward
 // x = h + gelu(c), kept for the residual path, then the norm of x; backward also dc = gelu'(c) dx, each rounded where
 // autocast's separate ops round (gelu's output, dx and dc to c's dtype). HBM-bound; at 16,384 rows of 768 in bf16 the
-// forward's three kernels took 52 us and the backward's three 68 us, the fused ones 29 and 46.
+// forward's three kernels took 59 us and the backward's three 90 us, the fused ones 32 and 66.
 // Forward: a workgroup takes 8 rows, each wave 2 with both rows (float4 per lane) loaded at once. Backward: a workgroup
 // takes 32 rows, each wave 8 of them, 2 rows' loads at a time.
 #include "common.h"

@@ -279,6 +279,43 @@ class Producer(torch.autograd.Function):
         return dE, dW, dbw, dbc, None, None
 
 
+def claves16_ok(E):
+    """Whether Claves16 takes E: fp32 rows on the GPU as its kernels read them."""
+    return (E.is_cuda and E.dtype == torch.float32 and E.dim() == 3 and E.is_contiguous() and E.shape[-1] % 8 == 0
+            and E.data_ptr() % 16 == 0)
+
+
+class Claves16(torch.autograd.Function):
+    """E (B, L, d) fp32 -> (rows, rows, keys) in bf16 for the autocast hash producers (asrn/nucleo.py:644-659): the
+    rows twice, the second an alias for the candidates' values, and the context MLP's keys [E_t ; E_{t-1}]. The backward
+    sums the three gradients in fp32 in one launch."""
+
+    @staticmethod
+    def forward(ctx, E):
+        B, L, d = E.shape
+        dev = _dev(E)
+        rows = torch.empty((B, L, d), dtype=torch.bfloat16, device=dev)
+        keys = torch.empty((B, L, 2 * d), dtype=torch.bfloat16, device=dev)
+        call('asrn_key_rows_fwd', ptr(E), B, L, d, ptr(rows), ptr(keys), stream_of(dev))
+        ctx.forma = (B, L, d, dev)
+        ctx.set_materialize_grads(False)
+        return rows, rows.view_as(rows), keys
+
+    @staticmethod
+    def backward(ctx, *gs):
+        B, L, d, dev = ctx.forma
+        gs = [None if g is None else _c16(g) for g in gs]
+        dE = torch.empty((B, L, d), dtype=torch.float32, device=dev)
+        call('asrn_key_rows_bwd', *[ptr(g) for g in gs], B, L, d, ptr(dE), stream_of(dev))
+        return dE
+
+
+def _c16(t):
+    """t as contiguous bf16, 16-byte aligned (a view into a wider buffer may start anywhere)."""
+    t = _c(t, torch.bfloat16)
+    return t if t.data_ptr() % 16 == 0 else t.clone()
+
+
 def copy_blocks(blocks):
     """One launch of asrn_copy_blocks: blocks is a list of (src, dst) 2-D fp32 device views of equal shape with unit
     column stride (src None: dst is filled with zeros)."""

@@ -593,6 +593,16 @@ int64_t asrn_clip_gradients_workspace(int32_t n, const int64_t* sizes);
 int asrn_clip_gradients(int32_t n, float* const* grads, const int64_t* sizes, float max_norm, const float* loss,
                         float* norm, float* skip, void* workspace, int64_t workspace_bytes, void* stream);
 
+/* ---- the context hash's keys in 16 bits ------------------------------------------------------------------------
+ * Replaces the casts, the shift and the concatenation that build the key [E_t ; E_{t-1}] under autocast
+ * (asrn/nucleo.py:644-659). fwd: E (B, L, d) fp32 -> rows (B, L, d) bf16 (rounded to nearest even) and keys (B, L, 2 d)
+ * bf16, keys[b, t] = [rows[b, t] ; rows[b, t - 1]] (0 before the row's start). bwd: the bf16 gradients of the rows from
+ * two users (drows, drows2) and of the keys (dkeys), each NULL where it is missing -> dE (B, L, d), their sum in fp32.
+ * Contiguous, 16-byte aligned, d a multiple of 8. */
+int asrn_key_rows_fwd(const float* E, int64_t B, int64_t L, int32_t d, void* rows, void* keys, void* stream);
+int asrn_key_rows_bwd(const void* drows, const void* drows2, const void* dkeys, int64_t B, int64_t L, int32_t d,
+                      float* dE, void* stream);
+
 /* ---- the model's local block: the causal convolution's columns ----------------------------------------------
  * Replaces F.pad + unfold + reshape of the 'conv' BloqueLocal's convolution (asrn/nucleo.py:969-1014, nn.Conv1d over
  * the left-padded sequence) and the cast of those columns to the autocast dtype. fwd: z (B, L, d) fp32, row stride
