@@ -408,8 +408,9 @@ SMALL_GEMM_MAX_MACS = 256 ** 3
 
 def _mm32(A, B, ta=False, tb=False):
     """fp32 op(A) @ op(B) (op the transpose where ta, tb) for the products past SMALL_GEMM_MAX_MACS: asrn_gemm, or the
-    library GEMM outside any autocast region where the sizes are not multiples of 4."""
-    if all(x % 4 == 0 for x in (*A.shape, *B.shape)):
+    library GEMM outside any autocast region where the sizes are not multiples of 4 or a matrix (a parameter that is a
+    view into a flat buffer) starts off a 16-byte boundary."""
+    if all(x % 4 == 0 for x in (*A.shape, *B.shape)) and A.data_ptr() % 16 == 0 and B.data_ptr() % 16 == 0:
         return gemm(A, ta, B, tb)
     with torch.autocast(device_type=A.device.type, enabled=False):
         return (A.t() if ta else A).mm(B.t() if tb else B)
@@ -1402,7 +1403,8 @@ def incrustar_ok(emb, x):
     return (w.is_cuda and x.device == w.device and x.dtype == torch.int64 and w.dtype == torch.float32 and w.requires_grad
             and torch.is_grad_enabled() and 1 <= x.numel() <= FICHAS_INCRUSTAR and type(emb) is torch.nn.Embedding
             and emb.padding_idx is None and emb.max_norm is None and not emb.scale_grad_by_freq and not emb.sparse
-            and not emb._forward_hooks and not emb._forward_pre_hooks and not emb._backward_hooks)
+            and not emb._forward_hooks and not emb._forward_pre_hooks and not emb._backward_hooks
+            and not emb._backward_pre_hooks)
 
 
 def incrustar(emb, x):

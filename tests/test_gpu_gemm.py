@@ -5,7 +5,7 @@ accumulator (K / 16 steps of six products): 2^-24 (2 + sqrt(K)) covers both in t
 import pytest
 import torch
 
-from asrn_amd import _lib
+from asrn_amd import _lib, ops
 from asrn_amd.lineal import gemm, lineal, weight_grad
 
 pytestmark = pytest.mark.gpu
@@ -117,3 +117,17 @@ def test_weight_gradient_in_a_graph():
         torch.cuda.synchronize()
         assert all(torch.equal(x, y) for x, y in zip(out, ref))
         gemm(a, True, b, False)
+
+
+def test_weights_off_a_16_byte_boundary():
+    """SmallMatmul past its own kernel's size on a weight that is a view into a flat buffer: the library GEMM takes it."""
+    g = torch.Generator(device='cuda').manual_seed(2)
+    n = 288
+    a = torch.randn(n * n + 1, generator=g, device='cuda')[1:].view(n, n).requires_grad_()
+    b = torch.randn(n, n, generator=g, device='cuda').requires_grad_()
+    gy = torch.randn(n, n, generator=g, device='cuda')
+    y = ops.SmallMatmul.apply(a, b)
+    da, db = torch.autograd.grad(y, (a, b), gy)
+    d = lambda t: t.detach().double()
+    for o, e in ((y, d(a) @ d(b)), (da, d(gy) @ d(b).t()), (db, d(a).t() @ d(gy))):
+        assert _rel(o.detach(), e) <= 2.0 ** -24 * (4 + n ** 0.5)

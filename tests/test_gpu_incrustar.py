@@ -24,3 +24,11 @@ def test_matches_torch(B, L, V, d, uno):
     ref = torch.zeros(V, d, dtype=torch.float64, device='cuda').index_add_(0, x.reshape(-1), gy.double().reshape(-1, d))
     mag = torch.zeros_like(ref).index_add_(0, x.reshape(-1), gy.double().abs().reshape(-1, d))
     assert bool(((dw.double() - ref).abs() <= 2.0 ** -24 * (B * L) ** 0.5 * mag + 1e-30).all())
+
+
+def test_backward_pre_hook_runs():
+    emb = torch.nn.Embedding(7, 8).cuda()
+    vistos = []
+    emb.register_full_backward_pre_hook(lambda m, g: vistos.append(tuple(g[0].shape)))
+    ops.incrustar(emb, torch.tensor([[1, 2, 2]], device='cuda')).sum().backward()
+    assert vistos == [(1, 3, 8)]
