@@ -66,10 +66,10 @@ __device__ __forceinline__ void split3(float x, float y, uint32_t (&p)[3]) {
 
 // One operand's share of a K step: R rows (of op(A), or columns of op(B)) by BK. T: stored with the rows contiguous
 // (element (k, r) at k * ld + r), else with k contiguous. A thread holds U units of 8 consecutive k.
-template <int R, bool T, bool F32, int BK>
+template <int R, bool T, bool F32, int BK, int THR = kGemmThr>
 struct Operand {
   static constexpr int CH = BK / 8;                          // units per row
-  static constexpr int U = R * CH / kGemmThr;                // units per thread
+  static constexpr int U = R * CH / THR;                     // units per thread
   static constexpr int PL = F32 ? 3 : 1;                     // bf16 planes
   // LDS unit of row r in chunk c: bank groups of 8 units. K-contiguous loads write units (c, r) with c fastest, CH to a
   // row: a chunk stride of 8 / CH mod 8 keeps 8 lanes apart. bf16 transposes write rows 4 apart: a spare unit every 8
@@ -88,7 +88,7 @@ struct Operand {
       c = tid / G;
       r = (tid % G) * U + i;
     } else {
-      const int u = tid + kGemmThr * i;
+      const int u = tid + THR * i;
       c = u % CH;
       r = u / CH;
     }
@@ -136,13 +136,7 @@ struct Operand {
         const int k = k0 + 8 * c + j;
         const bool ok = FULL || k < k1;
         const uint16_t* p = x + (int64_t)(ok ? k : k1 - 1) * ld + col;
-        if constexpr (U == 8) {
-          const uint2 v = *reinterpret_cast<const uint2*>(p), x2 = *reinterpret_cast<const uint2*>(p + 4);
-          w[j][0] = ok ? v.x : 0u;
-          w[j][1] = ok ? v.y : 0u;
-          w[j][2] = ok ? x2.x : 0u;
-          w[j][3] = ok ? x2.y : 0u;
-        } else if constexpr (U == 4) {
+        if constexpr (U == 4) {
           const uint2 v = *reinterpret_cast<const uint2*>(p);
           w[j][0] = ok ? v.x : 0u;
           w[j][1] = ok ? v.y : 0u;
@@ -338,6 +332,140 @@ __global__ __launch_bounds__(kGemmThr, 2) void k_gemm(Gemm g) {
   }
 }
 
+// The largest bf16 weight gradients: 256 x 256 tiles of 8 waves, 128 x 64 results each, one workgroup a CU. Wider wave
+// tiles read less LDS per product (with 64 x 64 a wave's reads and the stores take longer than its MFMA), and two LDS
+// buffers leave one barrier per 64 k: a step's loads are issued at its end and first waited for three quarters into the
+// next one's products (the scheduling barrier: the compiler would wait at once), split and stored between the rest.
+// With their sums (us, tiles of 256 x 128 or 128 x 128 / these): 768 x 3072 over 16384 tokens 134 / 120, 768 x 1536
+// 82 / 72, 512 x 2048 over 65536 240 / 187; 1536 x 768 over 8192 53.3 / 52.2, over 4097 38.7 / 42.4 (too few steps a
+// workgroup).
+constexpr int kWideThr = 512;
+__global__ __launch_bounds__(kWideThr, 2) void k_gemm_wide(Gemm g) {
+  constexpr int BM = 256, BN = 256, BK = 64, HEAD = 3;    // HEAD: 16-deep products before the loads are waited for
+  using O = Operand<256, true, false, BK, kWideThr>;
+  constexpr int WN = 4, MI = 4, NI = BN / WN / 32;
+  __shared__ uint4 lds[4 * O::UNITS];
+  const int total = g.tm * g.tn * g.splits, per = (total + kXcdCount - 1) / kXcdCount;
+  const int t = (int)(blockIdx.x % kXcdCount) * per + (int)(blockIdx.x / kXcdCount);
+  if (t >= total) return;
+  const int z = t / (g.tm * g.tn), tile = t % (g.tm * g.tn), bm = tile / g.tn, bn = tile % g.tn;
+  const int tid = threadIdx.x, lane = lane_id(), wave = tid >> 6;
+  const int m0 = bm * BM, n0 = bn * BN, ka = z * g.kper, kb = ka + g.kper < g.K ? ka + g.kper : g.K;
+  const int wm = wave / WN * 128, wn = wave % WN * (BN / WN), lr = lane & 31, lc = lane >> 5;
+  const bool sums = g.colsum != nullptr && bn == 0;
+  float cs[O::U];
+#pragma unroll
+  for (int i = 0; i < O::U; ++i) cs[i] = 0.f;
+  fx16 acc[MI][NI];
+#pragma unroll
+  for (int i = 0; i < MI; ++i)
+#pragma unroll
+    for (int j = 0; j < NI; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+  auto load = [&](O& a, O& b, int k) {
+    if (k + BK <= kb) {
+      a.template load<true>(g.A, g.lda, m0, g.M, k, kb, tid);
+      b.template load<true>(g.B, g.ldb, n0, g.N, k, kb, tid);
+    } else {
+      a.template load<false>(g.A, g.lda, m0, g.M, k, kb, tid);
+      b.template load<false>(g.B, g.ldb, n0, g.N, k, kb, tid);
+    }
+  };
+  uint4* l0 = lds;
+  uint4* l1 = lds + 2 * O::UNITS;
+  auto products = [&](int k0, int k1) {
+#pragma unroll
+    for (int kk = k0; kk < k1; ++kk) {
+      bfx8 fa[MI], fb[NI];
+#pragma unroll
+      for (int i = 0; i < MI; ++i) fa[i] = __builtin_bit_cast(bfx8, l0[O::at(0, 2 * kk + lc, wm + 32 * i + lr)]);
+#pragma unroll
+      for (int j = 0; j < NI; ++j)
+        fb[j] = __builtin_bit_cast(bfx8, l0[O::UNITS + O::at(0, 2 * kk + lc, wn + 32 * j + lr)]);
+#pragma unroll
+      for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int j = 0; j < NI; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[i], fb[j], acc[i][j], 0, 0, 0);
+    }
+  };
+  O a, b;
+  auto store = [&](uint4* l) {
+    a.template store<false>(l, tid);
+    b.template store<false>(l + O::UNITS, tid);
+    if (sums) a.column_sums(cs);
+  };
+  auto swap = [&]() {
+    uint4* x = l0;
+    l0 = l1;
+    l1 = x;
+  };
+  load(a, b, ka);                                 // kper > 0 and z < splits: ka < kb
+  store(l0);
+  if (ka + BK < kb) load(a, b, ka + BK);
+  __syncthreads();
+  int k = ka;
+  for (; k + 3 * BK <= kb; k += BK) {             // step k's products, step k + 1 to LDS, step k + 2 on its way
+    products(0, HEAD);
+    __builtin_amdgcn_sched_barrier(0);
+    products(HEAD, BK / 16);
+    store(l1);
+    a.template load<true>(g.A, g.lda, m0, g.M, k + 2 * BK, kb, tid);
+    b.template load<true>(g.B, g.ldb, n0, g.N, k + 2 * BK, kb, tid);
+    __syncthreads();
+    swap();
+  }
+  for (; k + BK < kb; k += BK) {
+    products(0, HEAD);
+    __builtin_amdgcn_sched_barrier(0);
+    products(HEAD, BK / 16);
+    store(l1);
+    if (k + 2 * BK < kb) load(a, b, k + 2 * BK);
+    __syncthreads();
+    swap();
+  }
+  products(0, BK / 16);
+  float* out = g.splits > 1 ? g.part + (int64_t)z * g.pstride : g.C;
+  const int64_t ldo = g.splits > 1 ? g.N : g.ldc;
+  const bool last = g.splits == 1;
+#pragma unroll
+  for (int i = 0; i < MI; ++i)
+#pragma unroll
+    for (int j = 0; j < NI; ++j) {
+      const int n = n0 + wn + 32 * j + lr;
+      const float bias = last && g.bias && n < g.N ? g.bias[n] : 0.f;
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const int m = m0 + wm + 32 * i + 8 * (e >> 2) + 4 * lc + (e & 3);
+        if (m < g.M && n < g.N) {
+          float* o = out + (int64_t)m * ldo + n;
+          float v = acc[i][j][e];
+          if (last) v += bias;
+          if (last && g.accumulate) v += *o;
+          *o = v;
+        }
+      }
+    }
+  if (sums) {                                     // uniform: the chunks' sums of a row combine in order
+    float* red = reinterpret_cast<float*>(lds);
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < O::U; ++i) {
+      int c, r;
+      O::where(tid, i, c, r);
+      red[c * BM + r] = cs[i];
+    }
+    __syncthreads();
+    if (tid < BM && m0 + tid < g.M) {
+      float v = 0.f;
+#pragma unroll
+      for (int c = 0; c < O::CH; ++c) v += red[c * BM + tid];
+      (last ? g.colsum : out + (int64_t)g.M * g.N)[m0 + tid] = v;
+    }
+  }
+}
+
 // C (+)= the sum of the partial products in split order (+ bias), and the column sums behind them. A workgroup takes
 // 32 float4 columns by 8 lanes of splits; the lanes combine in order.
 constexpr int kSumCols = 32, kSumLanes = kGemmThr / kSumCols;
@@ -391,18 +519,18 @@ static Plan plan_of(int64_t M, int64_t N, int64_t K, bool f32, int tile, int spl
   Plan p;
   if (tile) {
     p.bm = tile >> 8;
-    p.bn = tile & 255;
+    p.bn = tile & 255 ? tile & 255 : 256;
   } else {
     p.bm = p.bn = 64;
     const int64_t t128 = ((M + 127) / 128) * ((N + 127) / 128);
     if (M > 64 && N > 64 && (t128 >= 448 || (M * N >= 768 * 768 && K >= 2048))) p.bm = p.bn = 128;
-    if (!f32 && M % 8 == 0 && M * N >= 2 << 20) p.bm = 256;   // its threads take 8 columns of A
+    if (!f32 && M * N >= 1 << 20 && (M * N >= 2 << 20 || (double)M * N * K >= 9.6e9)) p.bm = p.bn = 256;
   }
   const int bk = !f32 || p.bm + p.bn == 128 ? 64 : 32;
   const int64_t tiles = ((M + p.bm - 1) / p.bm) * ((N + p.bn - 1) / p.bn);
   int64_t s = splits;
   if (s <= 0) {
-    s = 512 / tiles;
+    s = (p.bn == 256 ? 256 : 512) / tiles;
     const int64_t most = K <= 4096 ? K / 64 : K / 256;
     if (s > most) s = most;
     if (tiles >= 128 && K <= 1024) s = 1;
@@ -459,7 +587,7 @@ extern "C" int asrn_gemm(const void* A, int64_t lda, int32_t trans_a, const void
                    ((uintptr_t)bias & 15) == 0 && ((uintptr_t)colsum & 15) == 0, "asrn_gemm: misaligned operand");
   ASRN_REQUIRE(colsum == nullptr || ta, "asrn_gemm: column sums are those of A^T's A");
   ASRN_REQUIRE(tile == 0 || tile == (128 << 8 | 128) || tile == (64 << 8 | 128) || tile == (128 << 8 | 64) ||
-                   tile == (64 << 8 | 64) || (bf16 && M % 8 == 0 && tile == (256 << 8 | 128)), "asrn_gemm: unknown tile %d", tile);
+                   tile == (64 << 8 | 64) || (bf16 && tile == 256 << 8), "asrn_gemm: unknown tile %d", tile);
   const Plan p = plan_of(M, N, K, !bf16, tile, splits);
   Gemm g = {A, lda, B, ldb, C, ldc, (int)M, (int)N, (int)K, bias, accumulate ? 1 : 0, colsum, (float*)workspace,
             M * N + (colsum ? M : 0), p.splits, p.kper, (int)((M + p.bm - 1) / p.bm), (int)((N + p.bn - 1) / p.bn)};
@@ -472,7 +600,8 @@ extern "C" int asrn_gemm(const void* A, int64_t lda, int32_t trans_a, const void
   hipStream_t st = (hipStream_t)stream;
   const unsigned grid = (unsigned)((total + kXcdCount - 1) / kXcdCount * kXcdCount);
   if (bf16) {
-    if (p.bm == 256) launch_tile<256, 128, false>(ta, rows_b, g, grid, st);
+    if (p.bn == 256)
+      hipLaunchKernelGGL(k_gemm_wide, dim3(grid), dim3(kWideThr), 0, st, g);
     else if (p.bm == 128 && p.bn == 128) launch_tile<128, 128, false>(ta, rows_b, g, grid, st);
     else if (p.bm == 128) launch_tile<128, 64, false>(ta, rows_b, g, grid, st);
     else if (p.bn == 128) launch_tile<64, 128, false>(ta, rows_b, g, grid, st);

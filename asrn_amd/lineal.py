@@ -58,10 +58,15 @@ def _slab(t, s):
 MIN_PRODUCTO = 400_000_000
 # fp32 weight gradients over fewer tokens stay there too: 64 x 64 over 200 tokens 7.7 / 9.9, 64 x 256 over 2048 19.0 / 9.6
 MIN_FICHAS = 512
-# bf16 weight gradients on asrn_gemm: weights too large for slab copies (768 x 3072 over 16384 tokens 157 / 129,
-# 1536 x 768 124 / 80) and small ones (112 x 128 12.4 / 11.4, 64 x 1024 over 65536 34 / 32, 512 x 256 over 5008
+# bf16 weight gradients on asrn_gemm: weights too large for slab copies (768 x 3072 over 16384 tokens 154 / 120,
+# 1536 x 768 115 / 72) and small ones (112 x 128 12.4 / 11.4, 64 x 1024 over 65536 34 / 32, 512 x 256 over 5008
 # 18.7 / 15.1); between them hipBLASLt's batched slabs win (768 x 768 35 / 51, 512 x 512 over 65536 55 / 69)
 MAX_PESO_16 = 1 << 17
+# Of the large ones, only over enough tokens for their partial products: tokens times this at least the weight's elements,
+# with the bias gradient (13 us or more as a launch of its own) and without. 768 x 3072 with it over 2048 tokens 37 / 48,
+# over 5001 68 / 63, 512 x 2048 over 3000 41 / 33, 8000 x 512 over 8192 105 / 111; without it 768 x 3072 over 8192 77 / 81,
+# 1536 x 768 over 4097 35 / 39, over 8192 60 / 52, 32768 x 768 over 16384 763 / 1109
+FICHAS_PESO = {True: 400, False: 200}
 
 
 def _apto(t):
@@ -104,7 +109,9 @@ def _gradiente_ok(g2, x2, sesgo):
     n, peso = g2.shape[0], g2.shape[1] * x2.shape[1]
     if g2.dtype == torch.float32:
         return sesgo or n >= MIN_FICHAS
-    return peso >= MAX_SLAB_WEIGHT or peso <= MAX_PESO_16 or slabs_for(n, peso) == 1
+    if peso >= MAX_SLAB_WEIGHT:
+        return n * FICHAS_PESO[sesgo] >= peso
+    return peso <= MAX_PESO_16 or slabs_for(n, peso) == 1
 
 
 def _acc_dtype(t):

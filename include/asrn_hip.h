@@ -206,8 +206,8 @@ int asrn_column_sums(const void* x, int32_t bf16, int64_t rows, int64_t cols, in
  * into three bf16 parts whose products run on the matrix cores. bf16 != 0: bf16 operands, A stored (K, M) and B (K, N),
  * summed in fp32. colsum (M), with trans_a: also the sums of A's columns over K. N, M (trans_a) and K (an operand with
  * k contiguous) and the leading dimensions are multiples of 4, fp32 pointers 16-byte and bf16 ones 8-byte aligned.
- * tile: 0 (chosen by the sizes) or rows << 8 | columns of 64 or 128; splits: 0 (chosen) or the slabs of K summed in
- * order. workspace: asrn_gemm_workspace bytes (0: none needed). */
+ * tile: 0 (chosen by the sizes), rows << 8 | columns of 64 or 128, or for bf16 256 << 8 (256 x 256); splits: 0 (chosen)
+ * or the slabs of K summed in order. workspace: asrn_gemm_workspace bytes (0: none needed). */
 int64_t asrn_gemm_workspace(int64_t M, int64_t N, int64_t K, int32_t bf16, int32_t colsum, int32_t tile,
                             int32_t splits);
 int asrn_gemm(const void* A, int64_t lda, int32_t trans_a, const void* B, int64_t ldb, int32_t trans_b, int32_t bf16,

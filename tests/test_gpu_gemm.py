@@ -49,11 +49,9 @@ def test_fp32_matches_float64(tile, ta, tb, M, N, K):
         assert _rel(out[:, :N], exact + bias.double() + c0[:, :N].double()) <= bound + 2.0 ** -22
 
 
-@pytest.mark.parametrize('tile', TILES + [256 << 8 | 128])
-@pytest.mark.parametrize('M,N,K', [(8, 4, 1), (4, 8, 7), (136, 124, 65), (264, 136, 700)])
+@pytest.mark.parametrize('tile', TILES + [256 << 8])
+@pytest.mark.parametrize('M,N,K', [(8, 4, 1), (4, 8, 7), (136, 124, 65), (264, 136, 700), (260, 516, 64), (512, 260, 333)])
 def test_bf16_weight_gradient(tile, M, N, K):
-    if tile >> 8 == 256 and M % 8:
-        tile = 0
     g = torch.Generator(device='cuda').manual_seed(K)
     a = torch.randn(K, M, generator=g, device='cuda').bfloat16()
     b = torch.randn(K, N, generator=g, device='cuda').bfloat16()
