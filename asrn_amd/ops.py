@@ -13,7 +13,7 @@ import torch.nn.functional as F
 
 from . import _lib
 from ._lib import call, ptr, query, stream_of
-from .lineal import column_sums, gemm, gemm_ok, weight_grad
+from .lineal import column_sums, gemm, weight_grad
 
 I32 = torch.int32
 
@@ -215,14 +215,6 @@ class ContextProj(torch.autograd.Function):
 # a0 (the hash MLPs' first layers)
 # ---------------------------------------------------------------------------------------------------------------------
 
-def _sumar_producto(out, a, b):
-    """out += a @ b, fp32, in place."""
-    if gemm_ok(a, b, False) and out.data_ptr() % 16 == 0:
-        gemm(a, False, b, False, out=out, sumar=True)
-    else:
-        out.addmm_(a, b)
-
-
 class Producer(torch.autograd.Function):
     """y = E W^T by one bias-free GEMM, W's rows [W_p (m) | W_a (mc) | W_b (mc)]; returns the hash MLPs' hidden units
     g (B, L, m + mc) = [gelu(W_p E_t + b_word) | gelu(W_a E_t + W_b E_{t-1} + b_ctx)] (asrn_hidden_fwd;
@@ -270,7 +262,7 @@ class Producer(torch.autograd.Function):
             else:
                 # the rows' gradient is a fresh buffer of the candidate backward: accumulate the GEMM into it
                 dE = _c(drows, torch.float32) if drows.dtype != torch.float32 or not drows.is_contiguous() else drows
-                _sumar_producto(dE.view(B * L, d), dy2, W)
+                dE.view(B * L, d).addmm_(dy2, W)
         if ctx.needs_input_grad[1]:
             dW = weight_grad(dy2, E.view(B * L, d))
         if ctx.needs_input_grad[2] or ctx.needs_input_grad[3]:
@@ -396,7 +388,7 @@ class HashProducer(torch.autograd.Function):
             else:
                 # the rows' gradient is a fresh buffer of the candidate backward: accumulate the GEMM into it
                 dE = _c(drows, torch.float32) if drows.dtype != torch.float32 or not drows.is_contiguous() else drows
-                _sumar_producto(dE.view(B * L, d), dy2, W)
+                dE.view(B * L, d).addmm_(dy2, W)
         dW = weight_grad(dy2, E.view(B * L, d)) if ctx.needs_input_grad[1] else None
         return (dE, dW, dbw, dbc, dW2w.view(Pw, m), db2w, dW2c.view(Pc, mc), db2c, None, None, None, None)
 
