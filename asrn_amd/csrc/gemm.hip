@@ -44,6 +44,7 @@ struct Gemm {
   float* part;            // splits > 1: the partial products, one row of `pstride` floats per split
   int64_t pstride;
   int splits, kper, tm, tn;
+  int tail, tsplits, tkper;   // the last `tail` tiles are cut along K into tsplits slabs of tkper, summed by k_gemm_tail
 };
 
 // x, y (NEG: -x, -y) as three bf16 pairs, each the remainder's nearest
@@ -208,12 +209,17 @@ __global__ __launch_bounds__(kGemmThr, 2) void k_gemm(Gemm g) {
   uint4* la = lds;
   uint4* lb = lds + OA::UNITS;
   // XCD x takes a contiguous range of tiles, n fastest, then m, then the K slabs: tiles that share rows share its L2
-  const int total = g.tm * g.tn * g.splits, per = (total + kXcdCount - 1) / kXcdCount;
-  const int t = (int)(blockIdx.x % kXcdCount) * per + (int)(blockIdx.x / kXcdCount);
+  const int whole = g.tm * g.tn * g.splits - g.tail;                // a multiple of the XCDs when tail > 0
+  const int first = (whole + kXcdCount - 1) / kXcdCount * kXcdCount;
+  const bool cut = (int)blockIdx.x >= first;                          // a slab of a tail tile
+  const int total = cut ? g.tail * g.tsplits : whole, blk = (int)blockIdx.x - (cut ? first : 0);
+  const int per = (total + kXcdCount - 1) / kXcdCount, t = blk % kXcdCount * per + blk / kXcdCount;
   if (t >= total) return;
-  const int z = t / (g.tm * g.tn), tile = t % (g.tm * g.tn), bm = tile / g.tn, bn = tile % g.tn;
+  const int tiles = cut ? g.tail : g.tm * g.tn;
+  const int z = t / tiles, tile = t % tiles + (cut ? whole : 0), bm = tile / g.tn, bn = tile % g.tn;
+  const int kper = cut ? g.tkper : g.kper;
   const int tid = threadIdx.x, lane = lane_id(), wave = tid >> 6;
-  const int m0 = bm * BM, n0 = bn * BN, ka = z * g.kper, kb = ka + g.kper < g.K ? ka + g.kper : g.K;
+  const int m0 = bm * BM, n0 = bn * BN, ka = z * kper, kb = ka + kper < g.K ? ka + kper : g.K;
   const int wm = (wave >> 1) * (BM / 2), wn = (wave & 1) * (BN / 2), lr = lane & 31, lc = lane >> 5;
   const bool sums = TA && g.colsum != nullptr && bn == 0;
   float cs[OA::U];
@@ -269,9 +275,9 @@ __global__ __launch_bounds__(kGemmThr, 2) void k_gemm(Gemm g) {
               acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[i][pa], fb[j][q - pa], acc[i][j], 0, 0, 0);
     }
   }
-  float* out = g.splits > 1 ? g.part + (int64_t)z * g.pstride : g.C;
-  const int64_t ldo = g.splits > 1 ? g.N : g.ldc;
-  const bool last = g.splits == 1;
+  float* out = cut ? g.part + ((int64_t)t * BM - m0) * BN - n0 : g.splits > 1 ? g.part + (int64_t)z * g.pstride : g.C;
+  const int64_t ldo = cut ? BN : g.splits > 1 ? g.N : g.ldc;
+  const bool last = g.splits == 1 && !cut;
   uint64_t bad = 0;                               // results to form again (bit (i NI + j) 16 + e)
 #pragma unroll
   for (int i = 0; i < MI; ++i)
@@ -513,7 +519,32 @@ __global__ __launch_bounds__(kGemmThr) void k_gemm_sum(Gemm g) {
   *reinterpret_cast<float4*>(o) = s;
 }
 
-struct Plan { int bm, bn, splits, kper; };
+// The tail tiles: C (+)= the sum of their slabs in order (+ bias), one float4 a thread.
+__global__ __launch_bounds__(kGemmThr) void k_gemm_tail(Gemm g, int bm, int bn) {
+  const int e = ((int)blockIdx.x * kGemmThr + (int)threadIdx.x) * 4, size = bm * bn, tl = e / size, r = e - tl * size;
+  if (tl >= g.tail) return;
+  const int tile = g.tm * g.tn - g.tail + tl, m = tile / g.tn * bm + r / bn, n = tile % g.tn * bn + r % bn;
+  if (m >= g.M || n >= g.N) return;
+  float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
+  const float* p = g.part + e;
+  const int64_t stride = (int64_t)g.tail * size;
+#pragma unroll 4
+  for (int z = 0; z < g.tsplits; ++z) {
+    const float4 v = *reinterpret_cast<const float4*>(p + z * stride);
+    s.x += v.x; s.y += v.y; s.z += v.z; s.w += v.w;
+  }
+  float* o = g.C + (int64_t)m * g.ldc + n;
+  if (g.bias) { s.x += g.bias[n]; s.y += g.bias[n + 1]; s.z += g.bias[n + 2]; s.w += g.bias[n + 3]; }
+  if (g.accumulate) {
+    const float4 v = *reinterpret_cast<const float4*>(o);
+    s.x += v.x; s.y += v.y; s.z += v.z; s.w += v.w;
+  }
+  *reinterpret_cast<float4*>(o) = s;
+}
+
+struct Plan { int bm, bn, splits, kper, tail, tsplits, tkper; };
+
+constexpr int kSlots = 512;     // workgroups that run at once, 2 a CU
 
 static Plan plan_of(int64_t M, int64_t N, int64_t K, bool f32, int tile, int splits) {
   Plan p;
@@ -540,6 +571,20 @@ static Plan plan_of(int64_t M, int64_t N, int64_t K, bool f32, int tile, int spl
   if (s > steps) s = steps > 0 ? steps : 1;
   p.kper = (int)((steps + s - 1) / s) * bk;
   p.splits = (int)((K + p.kper - 1) / p.kper);
+  // A second round that fills less than half of the slots leaves most CUs idle: its tiles are cut along K over all of
+  // them (12000 x 768 x 3072, 564 tiles: 354 -> 303 us; 12000 x 768 x 1536 178 -> 155; 9000 x 1024 x 512 68 -> 61).
+  // Past two rounds it gains nothing (12000 x 1536 x 768, 1128 tiles: 162 -> 164 us).
+  p.tail = p.tsplits = p.tkper = 0;
+  const int64_t left = tiles % kSlots;
+  if (f32 && splits == 0 && p.splits == 1 && tiles > kSlots && tiles < 2 * kSlots) {
+    int64_t ts = kSlots / left;
+    if (ts > K / 128) ts = K / 128;
+    if (ts > 1) {
+      p.tkper = (int)((steps + ts - 1) / ts) * bk;
+      p.tsplits = (int)((K + p.tkper - 1) / p.tkper);
+      p.tail = (int)left;
+    }
+  }
   return p;
 }
 
@@ -563,6 +608,7 @@ extern "C" int64_t asrn_gemm_workspace(int64_t M, int64_t N, int64_t K, int32_t 
   if (M < 0 || N < 0 || K < 0) return -1;
   if (M == 0 || N == 0) return 0;
   const Plan p = plan_of(M, N, K, !bf16, tile, splits);
+  if (p.tail && !colsum) return (int64_t)p.tail * p.tsplits * p.bm * p.bn * 4;
   return p.splits > 1 ? (int64_t)p.splits * (M * N + (colsum ? M : 0)) * 4 : 0;
 }
 
@@ -588,17 +634,25 @@ extern "C" int asrn_gemm(const void* A, int64_t lda, int32_t trans_a, const void
   ASRN_REQUIRE(colsum == nullptr || ta, "asrn_gemm: column sums are those of A^T's A");
   ASRN_REQUIRE(tile == 0 || tile == (128 << 8 | 128) || tile == (64 << 8 | 128) || tile == (128 << 8 | 64) ||
                    tile == (64 << 8 | 64) || (bf16 && tile == 256 << 8), "asrn_gemm: unknown tile %d", tile);
-  const Plan p = plan_of(M, N, K, !bf16, tile, splits);
+  Plan p = plan_of(M, N, K, !bf16, tile, splits);
+  if (colsum) p.tail = 0;                                  // only whole tiles sum A's columns
   Gemm g = {A, lda, B, ldb, C, ldc, (int)M, (int)N, (int)K, bias, accumulate ? 1 : 0, colsum, (float*)workspace,
-            M * N + (colsum ? M : 0), p.splits, p.kper, (int)((M + p.bm - 1) / p.bm), (int)((N + p.bn - 1) / p.bn)};
+            M * N + (colsum ? M : 0), p.splits, p.kper, (int)((M + p.bm - 1) / p.bm), (int)((N + p.bn - 1) / p.bn),
+            p.tail, p.tsplits, p.tkper};
   const int64_t total = (int64_t)g.tm * g.tn * g.splits;
   ASRN_REQUIRE(total < (1 << 30), "asrn_gemm: too many tiles");
   if (p.splits > 1)
     ASRN_REQUIRE(workspace && workspace_bytes >= p.splits * g.pstride * 4 && ((uintptr_t)workspace & 15) == 0,
                  "asrn_gemm: needs a 16-byte aligned workspace of %lld bytes (got %lld)",
                  (long long)(p.splits * g.pstride * 4), (long long)workspace_bytes);
+  const int64_t slabs = (int64_t)p.tail * p.tsplits, slab_bytes = slabs * p.bm * p.bn * 4;
+  if (p.tail)
+    ASRN_REQUIRE(workspace && workspace_bytes >= slab_bytes && ((uintptr_t)workspace & 15) == 0,
+                 "asrn_gemm: needs a 16-byte aligned workspace of %lld bytes (got %lld)", (long long)slab_bytes,
+                 (long long)workspace_bytes);
   hipStream_t st = (hipStream_t)stream;
-  const unsigned grid = (unsigned)((total + kXcdCount - 1) / kXcdCount * kXcdCount);
+  auto blocks = [](int64_t n) { return (n + kXcdCount - 1) / kXcdCount * kXcdCount; };
+  const unsigned grid = (unsigned)(blocks(total - p.tail) + blocks(slabs));
   if (bf16) {
     if (p.bn == 256)
       hipLaunchKernelGGL(k_gemm_wide, dim3(grid), dim3(kWideThr), 0, st, g);
@@ -613,6 +667,11 @@ extern "C" int asrn_gemm(const void* A, int64_t lda, int32_t trans_a, const void
     else launch_tile<64, 64, true>(ta, rows_b, g, grid, st);
   }
   int rc = check_launch("asrn_gemm");
+  if (rc == 0 && p.tail) {
+    hipLaunchKernelGGL(k_gemm_tail, dim3((unsigned)(p.tail * (p.bm * p.bn / 4 / kGemmThr))), dim3(kGemmThr), 0, st, g, p.bm,
+                       p.bn);
+    return check_launch("asrn_gemm");
+  }
   if (rc || p.splits == 1) return rc;
   const int64_t cols = (g.pstride + 4 * kSumCols - 1) / (4 * kSumCols);
   hipLaunchKernelGGL(k_gemm_sum, dim3((unsigned)cols), dim3(kGemmThr), 0, st, g);

@@ -54,7 +54,7 @@ def _slab(t, s):
 
 # fp32 products of fewer multiply-adds than this stay on hipBLASLt, measured (us, it / asrn_gemm): 2048 x 64 x 256
 # 5.9 / 9.1, 4611 x 384 x 192 10.7 / 11.3, 5005 x 256 x 512 19.1 / 17.8, 4611 x 384 x 384 17.6 / 16.0, 32768 x 256 x 256
-# 39.1 / 33.1, 12000 x 768 x 3072 411 / 349: below, a launch's few steps wait for their loads
+# 39.1 / 33.1, 12000 x 768 x 3072 492 / 303: below, a launch's few steps wait for their loads
 MIN_PRODUCTO = 400_000_000
 # fp32 weight gradients over fewer tokens stay there too: 64 x 64 over 200 tokens 7.7 / 9.9, 64 x 256 over 2048 19.0 / 9.6
 MIN_FICHAS = 512

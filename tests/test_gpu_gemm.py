@@ -129,3 +129,19 @@ def test_weights_off_a_16_byte_boundary():
     d = lambda t: t.detach().double()
     for o, e in ((y, d(a) @ d(b)), (da, d(gy) @ d(b).t()), (db, d(a).t() @ d(gy))):
         assert _rel(o.detach(), e) <= 2.0 ** -24 * (4 + n ** 0.5)
+
+
+@pytest.mark.parametrize('tb,M,N,K', [(1, 4500, 1924, 260), (0, 4229, 2180, 516), (1, 8193, 1028, 388)])
+def test_tail_tiles_cut_along_k(tb, M, N, K):
+    """A little more than one round of 512 tiles of 128 x 128: the second round's tiles go through the workspace."""
+    g = torch.Generator(device='cuda').manual_seed(M)
+    r = lambda *s: torch.randn(*s, generator=g, device='cuda')
+    a, b, bias, c0 = r(M, K), r(N, K) if tb else r(K, N), r(N), r(M, N + 4)
+    assert 512 < -(-M // 128) * -(-N // 128) < 768 and _lib.query('asrn_gemm_workspace', M, N, K, 0, 0, 0, 0) > 0
+    a[M - 1, 3] = float('inf')
+    exact = a.double() @ (b.double().t() if tb else b.double())
+    out = c0.clone()
+    _llamar(a, 0, b, tb, M, N, K, out, 0, 0, bias=bias, accumulate=1)
+    assert torch.equal(out[M - 1, :N], (exact[M - 1] + bias + c0[M - 1, :N]).float())
+    assert _rel(out[:M - 1, :N], (exact + bias + c0[:, :N])[:M - 1]) <= 2.0 ** -24 * (2 + K ** 0.5) + 2.0 ** -22
+    assert torch.equal(out[:, N:], c0[:, N:])
