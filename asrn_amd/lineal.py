@@ -77,9 +77,13 @@ def _apto(t):
 
 def gemm(a, ta, b, tb, out=None, sesgo=None, sumar=False, columnas=False):
     """op(a) op(b) (+ sesgo) in fp32 on asrn_gemm, op the transpose where ta, tb; sumar: added into out. columnas (ta):
-    returns (product, the sums of a's columns)."""
+    returns (product, the sums of a's columns). Shapes that do not chain are refused here: the kernels see leading
+    dimensions only and would read whatever lies there."""
     M, K = (a.shape[1], a.shape[0]) if ta else a.shape
-    N = b.shape[0] if tb else b.shape[1]
+    Kb, N = (b.shape[1], b.shape[0]) if tb else b.shape
+    if K != Kb or (sesgo is not None and tuple(sesgo.shape) != (N,)):
+        raise ValueError(f'gemm: shapes {tuple(a.shape)}{" transposed" if ta else ""}, {tuple(b.shape)}'
+                         f'{" transposed" if tb else ""} and bias {None if sesgo is None else tuple(sesgo.shape)} do not chain')
     bf = int(a.dtype == torch.bfloat16)
     if out is None:
         out = torch.empty((M, N), dtype=torch.float32, device=a.device)
@@ -93,12 +97,15 @@ def gemm(a, ta, b, tb, out=None, sesgo=None, sumar=False, columnas=False):
 
 
 def gemm_ok(a, b, tb, sesgo=None):
-    """Whether a @ op(b) (+ sesgo) runs on asrn_gemm: fp32 on the GPU, aligned, MIN_PRODUCTO multiply-adds or more."""
+    """Whether a @ op(b) (+ sesgo) runs on asrn_gemm: fp32 on the GPU, aligned, MIN_PRODUCTO multiply-adds or more, and
+    shapes that chain with one bias value per column (F.linear broadcasts a bias or refuses the rest)."""
+    if b.dim() != 2 or a.shape[1] != b.shape[1 if tb else 0]:
+        return False
     (M, K), N = a.shape, b.shape[0 if tb else 1]
     return (a.is_cuda and a.dtype == b.dtype == torch.float32 and b.device == a.device and M * N * K >= MIN_PRODUCTO
             and max(M, N, K) < 1 << 30 and N >= 64 and N % 4 == 0 and K % 4 == 0 and _apto(a) and _apto(b)
-            and (sesgo is None or (sesgo.dtype == torch.float32 and sesgo.device == a.device and sesgo.is_contiguous()
-                                   and sesgo.data_ptr() % 16 == 0)))
+            and (sesgo is None or (sesgo.dtype == torch.float32 and sesgo.device == a.device and tuple(sesgo.shape) == (N,)
+                                   and sesgo.is_contiguous() and sesgo.data_ptr() % 16 == 0)))
 
 
 def _gradiente_ok(g2, x2, sesgo):

@@ -145,3 +145,24 @@ def test_tail_tiles_cut_along_k(tb, M, N, K):
     assert torch.equal(out[M - 1, :N], (exact[M - 1] + bias + c0[M - 1, :N]).float())
     assert _rel(out[:M - 1, :N], (exact + bias + c0[:, :N])[:M - 1]) <= 2.0 ** -24 * (2 + K ** 0.5) + 2.0 ** -22
     assert torch.equal(out[:, N:], c0[:, N:])
+
+
+@pytest.mark.parametrize('fin,fw,nb', [(512, 768, None), (768, 512, None), (512, 512, 1020), (512, 512, 4)])
+def test_shapes_that_do_not_chain_are_refused(fin, fw, nb):
+    """Products past MIN_PRODUCTO whose inner sizes differ, or whose bias is shorter than a row: F.linear's error."""
+    x, w = torch.ones(2, 512, fin, device='cuda'), torch.ones(1024, fw, device='cuda')
+    b = None if nb is None else torch.ones(nb, device='cuda')
+    with pytest.raises(RuntimeError):
+        torch.nn.functional.linear(x, w, b)
+    with pytest.raises(RuntimeError):
+        lineal(x, w, b)
+
+
+def test_a_bias_of_one_element_is_broadcast():
+    g = torch.Generator(device='cuda').manual_seed(3)
+    r = lambda *s: torch.randn(*s, generator=g, device='cuda').requires_grad_()
+    x, w, b, gy = r(2, 512, 512), r(1024, 512), r(1), r(2, 512, 1024).detach()
+    got, ref = lineal(x, w, b), torch.nn.functional.linear(x, w, b)
+    assert _rel(got.detach(), ref.detach().double()) <= 2.0 ** -24 * (4 + 512 ** 0.5)
+    gb, = torch.autograd.grad(got, b, gy)
+    assert gb.shape == b.shape and abs(gb.item() - gy.double().sum().item()) <= 2.0 ** -24 * 1024 * gy.abs().sum((0, 1)).norm().item()

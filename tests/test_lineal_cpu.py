@@ -4,7 +4,7 @@ import pytest
 import torch
 import torch.nn.functional as F
 
-from asrn_amd.lineal import lineal, slabs_for
+from asrn_amd.lineal import gemm, lineal, slabs_for
 
 
 def test_slab_counts():
@@ -40,3 +40,10 @@ def test_lineal_matches_linear(lead, fin, fout, bias, strided):
     for a, b_ in zip(leaves[0], leaves[1]):
         if a is not None:
             torch.testing.assert_close(b_.grad, a.grad, rtol=1e-10, atol=1e-10)
+
+
+@pytest.mark.parametrize('a,ta,b,tb,sesgo', [((8, 12), False, (16, 8), False, None), ((8, 12), False, (8, 16), True, None),
+                                             ((12, 8), True, (16, 8), False, None), ((8, 12), False, (12, 8), False, 4)])
+def test_gemm_refuses_shapes_that_do_not_chain(a, ta, b, tb, sesgo):
+    with pytest.raises(ValueError, match='do not chain'):
+        gemm(torch.zeros(a), ta, torch.zeros(b), tb, sesgo=None if sesgo is None else torch.zeros(sesgo))
