@@ -114,6 +114,8 @@ def _gradiente_ok(g2, x2, sesgo):
             and _apto(x2) and g2.shape[1] % 4 == 0 and x2.shape[1] % 4 == 0 and 1 <= g2.shape[0] < 1 << 30):
         return False
     n, peso = g2.shape[0], g2.shape[1] * x2.shape[1]
+    if peso == 0:                      # no product to form, but the bias gradient still is (asrn_gemm returns at once)
+        return False
     if g2.dtype == torch.float32:
         return sesgo or n >= MIN_FICHAS
     if peso >= MAX_SLAB_WEIGHT:

@@ -166,3 +166,16 @@ def test_a_bias_of_one_element_is_broadcast():
     assert _rel(got.detach(), ref.detach().double()) <= 2.0 ** -24 * (4 + 512 ** 0.5)
     gb, = torch.autograd.grad(got, b, gy)
     assert gb.shape == b.shape and abs(gb.item() - gy.double().sum().item()) <= 2.0 ** -24 * 1024 * gy.abs().sum((0, 1)).norm().item()
+
+
+@pytest.mark.parametrize('dt', [torch.float32, torch.bfloat16])
+def test_no_input_features(dt):
+    """A weight without columns (x a zero-wide view of aligned rows): the bias's gradient is still gy's column sums."""
+    x = torch.ones(700, 8, device='cuda', dtype=dt)[:, :0]
+    w = torch.zeros(64, 0, device='cuda', dtype=dt, requires_grad=True)
+    b = torch.zeros(64, device='cuda', dtype=dt, requires_grad=True)
+    gy = torch.ones(700, 64, device='cuda', dtype=dt)
+    poison = torch.full((1 << 20,), 7.0, device='cuda')
+    del poison
+    gw, gb = torch.autograd.grad(lineal(x, w, b), (w, b), gy)
+    assert gw.shape == w.shape and bool((gb == 700).all())
