@@ -13,6 +13,8 @@ On the GPU, the sums (the slab partials, and the bias gradients' column sums) ru
 (fp32 accumulation in a fixed order, no memset-cleared semaphores, safe to capture in a HIP graph). fp64 operands,
 and CPU tensors (the math checked on the CPU), use torch's sums.
 """
+import math
+
 import torch
 import torch.nn.functional as F
 
@@ -38,12 +40,13 @@ def _rows(t):
     """(N, k) view of a (..., k) tensor whose last axis is contiguous; copies only when the leading axes do not
     flatten to one stride."""
     k = t.shape[-1]
+    n = math.prod(t.shape[:-1])                      # stated: -1 has no value for a zero-wide t
     if t.stride(-1) != 1:
         t = t.contiguous()
     try:
-        return t.view(-1, k)
+        return t.view(n, k)
     except RuntimeError:
-        return t.reshape(-1, k)
+        return t.reshape(n, k)
 
 
 def _slab(t, s):

@@ -47,3 +47,11 @@ def test_lineal_matches_linear(lead, fin, fout, bias, strided):
 def test_gemm_refuses_shapes_that_do_not_chain(a, ta, b, tb, sesgo):
     with pytest.raises(ValueError, match='do not chain'):
         gemm(torch.zeros(a), ta, torch.zeros(b), tb, sesgo=None if sesgo is None else torch.zeros(sesgo))
+
+
+def test_no_input_features():
+    x, w, b = torch.ones(5, 3, 0), torch.zeros(4, 0, requires_grad=True), torch.ones(4, requires_grad=True)
+    y = lineal(x, w, b)
+    assert torch.equal(y, torch.ones(5, 3, 4))
+    gw, gb = torch.autograd.grad(y.sum(), (w, b))
+    assert gw.shape == (4, 0) and bool((gb == 15).all())
