@@ -4,7 +4,7 @@ with a ragged tail, against F.cross_entropy in float64. The tolerance is test_cr
 import pytest
 import torch
 
-from asrn_amd import ops
+from asrn_amd import _lib, ops
 
 pytestmark = pytest.mark.gpu
 
@@ -38,3 +38,21 @@ def test_no_rows_and_all_ignored():
     loss /= 2                                       # in place, before the backward
     loss.backward()
     assert torch.isfinite(x.grad).all()
+
+
+@pytest.mark.parametrize('rows', [1, 9, 1025, 8192, 70001])
+def test_reduction_rounds_once(rows):
+    """The rows' sum and mean against float64: summed in double, so one rounding (2^-24) of the exact result."""
+    g = torch.Generator(device='cuda').manual_seed(rows)
+    per = 9 + torch.randn(rows, generator=g, device='cuda')
+    y = torch.arange(rows, device='cuda')
+    per[rows // 2] = 0.0
+    y[rows // 2] = -100
+    n = rows - 1
+    for mean in (0, 1):
+        out, count = torch.empty((), device='cuda'), torch.empty((), device='cuda')
+        _lib.call('asrn_cross_entropy_reduce', _lib.ptr(per), _lib.ptr(y), rows, -100, mean, _lib.ptr(out),
+                  _lib.ptr(count), _lib.stream_of(per.device))
+        exact = per.double().sum() / (n if mean else 1)
+        assert count.item() == (n if mean else 1)
+        assert (n == 0 and mean and torch.isnan(out)) or abs(out.item() - exact.item()) <= 2.0 ** -24 * exact.item()
