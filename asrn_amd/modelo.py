@@ -123,7 +123,7 @@ class BloqueLocal(nn.Module):
             c = conv_causal(z, self.conv.weight, self.conv.bias)
         else:
             c = conv_canal_causal(z, self.conv.weight, self.conv.bias)
-        if self.mezcla == 'conv' and not (self.drop.training and self.drop.p > 0):
+        if self.mezcla == 'conv' and self._sin_drop():
             y, h = ops.suma_gelu_norma(self.ln2, h, c, _dtype_producto(h))
             return h + self._ff(y)
         c = F.gelu(c)
@@ -132,6 +132,12 @@ class BloqueLocal(nn.Module):
         h = h + self.drop(c)
         y, h = ops.norma_residual(self.ln2, h, _dtype_producto(h))
         return h + self.drop(self._ff(y))
+
+    def _sin_drop(self):
+        """Whether self.drop leaves everything as it is and its calls may be left out: a plain nn.Dropout (a module put
+        in its place has its own forward, and need not have p), inactive, without hooks."""
+        d = self.drop
+        return type(d) is nn.Dropout and not (d.training and d.p > 0) and ops.sin_ganchos(d)
 
     def _ff(self, y):
         """self.ff on the library's Linear (lineal: the bias gradients as the library's fixed-order column sums)."""

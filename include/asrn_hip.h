@@ -566,8 +566,8 @@ int asrn_block_finish_norm(const float* prev_h1, const float* prev_b2, const flo
  * training loop (asrn/nucleo.py:1108, 2301): the same fp32 arithmetic on fp32 or bf16 logits (logits_bf16), without
  * the fp32 copy of the logits. logits (rows, V) with row stride ld (16-byte aligned rows), target (rows) int64.
  * fwd: lse (rows) = logsumexp of the row, loss (rows) = lse - logits[target] (0 where target == ignore_index, NaN
- * for a target outside [0, V)). reduce: *out = the sum of the rows' losses (in double, rounded once), over the count of rows not ignored with
- * mean (NaN when there is none); *count = that count (1 without mean).
+ * for a target outside [0, V)). reduce: *out = the sum of the rows' losses (in double, rounded once), over the count
+ * of rows not ignored with mean (NaN when there is none); *count = that count (1 without mean).
  * bwd: dlogits (rows, V), row stride ldd, in the logits' dtype = (softmax - onehot(target)) * *scale / *count (device
  * floats: the loss's gradient and reduce's count, which may be null), 0 for ignored rows; bf16 rounded to nearest
  * even. */

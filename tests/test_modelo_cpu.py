@@ -294,3 +294,33 @@ def test_public_names_mirror_the_reference():
         assert hasattr(asrn_amd, n), n
     assert asrn_amd.load is asrn_amd.cargar and asrn_amd.train is asrn_amd.entrenar
     assert asrn_amd.MULT_SUFIJO_Y_PUERTA == 3.0
+
+
+class _Mitad(torch.nn.Module):
+    """A module in the dropout's place without p: halves what it is given."""
+
+    def forward(self, x):
+        return 0.5 * x
+
+
+@pytest.mark.parametrize('train', [True, False])
+def test_block_calls_what_stands_for_its_dropout(train):
+    torch.manual_seed(0)
+    b = asrn_amd.BloqueLocal(8, ff=16).train(train)
+    h = torch.randn(2, 5, 8)
+    base = b(h)
+    vistas = []
+    gancho = b.drop.register_forward_hook(lambda m, a, y: vistas.append(y.shape))
+    assert torch.equal(b(h), base) and vistas == [h.shape, h.shape]
+    gancho.remove()
+    en_todos = torch.nn.modules.module.register_module_forward_hook(
+        lambda m, a, y: vistas.append(None) if m is b.drop else None)
+    b(h)
+    en_todos.remove()
+    assert vistas[2:] == [None, None]
+    b.drop = torch.nn.Identity()
+    assert torch.equal(b(h), base)
+    b.drop = _Mitad()
+    c = conv_causal(b.ln1(h), b.conv.weight, b.conv.bias)
+    h1 = h + 0.5 * F.gelu(c)
+    torch.testing.assert_close(b(h), h1 + 0.5 * b.ff(b.ln2(h1)))
