@@ -1396,14 +1396,13 @@ class Incrustar(torch.autograd.Function):
 
 
 def incrustar_ok(emb, x):
-    """Whether incrustar(emb, x) runs asrn_embedding_bwd: a plain fp32 nn.Embedding in training on the GPU, up to
-    FICHAS_INCRUSTAR int64 tokens."""
+    """Whether incrustar(emb, x) runs asrn_embedding_bwd: a plain fp32 nn.Embedding in training on the GPU, whose call
+    is its class's forward and no hooks, up to FICHAS_INCRUSTAR int64 tokens."""
     w = emb.weight
     return (w.is_cuda and x.device == w.device and x.dtype == torch.int64 and w.dtype == torch.float32 and w.requires_grad
             and torch.is_grad_enabled() and 1 <= x.numel() <= FICHAS_INCRUSTAR and type(emb) is torch.nn.Embedding
             and emb.padding_idx is None and emb.max_norm is None and not emb.scale_grad_by_freq and not emb.sparse
-            and not emb._forward_hooks and not emb._forward_pre_hooks and not emb._backward_hooks
-            and not emb._backward_pre_hooks)
+            and sin_ganchos(emb))
 
 
 def incrustar(emb, x):

@@ -32,3 +32,21 @@ def test_backward_pre_hook_runs():
     emb.register_full_backward_pre_hook(lambda m, g: vistos.append(tuple(g[0].shape)))
     ops.incrustar(emb, torch.tensor([[1, 2, 2]], device='cuda')).sum().backward()
     assert vistos == [(1, 3, 8)]
+
+
+def test_global_hooks_and_a_replaced_forward_run():
+    emb = torch.nn.Embedding(7, 8).cuda()
+    x = torch.tensor([[1, 2, 2]], device='cuda')
+    assert ops.incrustar_ok(emb, x)
+    modulo = torch.nn.modules.module
+    for registrar in (modulo.register_module_forward_pre_hook, modulo.register_module_forward_hook,
+                      modulo.register_module_full_backward_pre_hook, modulo.register_module_full_backward_hook):
+        vistos = []
+        gancho = registrar(lambda m, *a: vistos.append(m))
+        try:
+            ops.incrustar(emb, x).sum().backward()
+        finally:
+            gancho.remove()
+        assert vistos == [emb]
+    emb.forward = lambda x: 2 * torch.nn.functional.embedding(x, emb.weight)
+    assert torch.equal(ops.incrustar(emb, x), 2 * emb.weight[x])
