@@ -24,11 +24,20 @@ MEZCLAS = ('conv', 'memoria')
 OPCIONES_CAPA = ('n_tablas', 'n_bits', 'afin_oculto', 'chunk', 'tablas_contexto', 'confirmar', 'sufijo', 'vistos',
                  'nodos_racha', 'racha_max')
 MODOS_CHECKPOINT = ('no', 'asrn', 'todo')
-# Embedding values (B L d) up to which a model's training step keeps its ASRN layers on one stream: a captured step
+# Embedding values (B L d) up to which a model's training step keeps its ASRN layers on one stream. A captured step
 # without branches replays with its launches back to back, one with a branch pays for them one by one, and below this
 # the launches cost more than the layers' two branches gain by running side by side (us a step, two streams / one: 512
-# tokens at d 64 690 / 599, 4096 at d 64 785 / 723, 4096 at d 256 1365 / 1324, 4096 at d 512 2588 / 2603)
+# tokens at d 64 690 / 599, 4096 at d 64 785 / 723, 4096 at d 256 1365 / 1324, 4096 at d 512 2588 / 2603); an eager step is bound
+# by the host and saves the second stream's events (4096 at d 64 3927 / 3606, at d 256 3644 / 3346). Only where the
+# embedding's gradient is the library's too (ops.incrustar_ok): torch's for longer batches, replayed back to back in a graph
+# without branches, ended in an illegal access in its own partition kernel (16 x 1024 tokens, d 64), cause not known.
 UNA_CORRIENTE = 1 << 20
+
+
+def _entiende_una(capa):
+    """Whether a call of the layer reaches CapaASRNEstable.forward itself: a wrapper or a replaced forward in its place
+    takes forward's other arguments, not the models' own una_corriente."""
+    return type(capa).forward is CapaASRNEstable.forward and 'forward' not in vars(capa)
 
 
 def _base(modelo):
@@ -221,11 +230,11 @@ class ModeloASRN(nn.Module):
             h = torch.utils.checkpoint.checkpoint(bloque, h, use_reentrant=False) if ck_bloque else bloque(h)
             if i in self.pos_largo:
                 capa = next(capas)
+                extra = {'una_corriente': True} if una and _entiende_una(capa) else {}
                 if ck_capa:
-                    h = torch.utils.checkpoint.checkpoint(capa, E, h, x, use_reentrant=False, ngramas=ng,
-                                                          una_corriente=una)
+                    h = torch.utils.checkpoint.checkpoint(capa, E, h, x, use_reentrant=False, ngramas=ng, **extra)
                 else:
-                    h = capa(E, h, x, ngramas=ng, una_corriente=una)
+                    h = capa(E, h, x, ngramas=ng, **extra)
         return h
 
     def forward(self, x):

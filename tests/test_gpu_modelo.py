@@ -20,7 +20,7 @@ import torch
 from safetensors import safe_open
 
 import asrn_amd
-from asrn_amd import archivo, synth
+from asrn_amd import archivo, modelo, synth
 
 pytestmark = pytest.mark.gpu
 DEV = 'cuda'
@@ -368,3 +368,62 @@ def test_configs3_model_step_bf16():
     print('losses on one batch', perdidas, flush=True)
     assert all(torch.isfinite(torch.tensor(perdidas)))
     assert perdidas[-1] < perdidas[0]
+
+
+class _Envoltura(torch.nn.Module):
+    """A layer's wrapper that takes the layer's documented arguments only."""
+
+    def __init__(self, capa):
+        super().__init__()
+        self.capa = capa
+
+    def __getattr__(self, nombre):
+        try:
+            return super().__getattr__(nombre)
+        except AttributeError:
+            return getattr(self.capa, nombre)
+
+    def forward(self, E, h, piezas=None, ngramas=None):
+        return self.capa(E, h, piezas, ngramas=ngramas)
+
+
+def _paso_pequeno(B, L, d, cambio=None):
+    m = asrn_amd.crear_modelo(97, d=d, n_capas=2, semilla=3, **REDUCIDA).to(DEV).train()
+    if cambio:
+        cambio(m)
+    w = synth.tokens(B, L + 1, 97, seed=4).to(DEV)
+    perdida = m.perdida(w[:, :-1].contiguous(), w[:, 1:].contiguous())
+    return [perdida.detach(), *torch.autograd.grad(perdida, list(m.parameters()))]
+
+
+@pytest.mark.parametrize('modo', ['envoltura', 'forward', 'subclase'])
+def test_layers_with_forwards_own_arguments_train_small_batches(modo):
+    """What a program put in a layer's place gets forward's arguments and no others, one stream or two."""
+    def cambio(m):
+        capa = m.largos[0]
+        if modo == 'envoltura':
+            m.largos[0] = _Envoltura(capa)
+        elif modo == 'forward':
+            capa.forward = lambda E, h, piezas=None, ngramas=None: type(capa).forward(capa, E, h, piezas, ngramas)
+        else:
+            capa.__class__ = type('Sub', (type(capa),), {
+                'forward': lambda s, E, h, piezas=None, ngramas=None: asrn_amd.CapaASRNEstable.forward(s, E, h, piezas,
+                                                                                                    ngramas)})
+    for a, b in zip(_paso_pequeno(2, 100, 64, cambio), _paso_pequeno(2, 100, 64)):
+        assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize('B,L,d,una', [(3, 171, 64, True), (4, 1000, 260, True), (4, 1000, 264, False)])
+def test_one_stream_and_two_agree(B, L, d, una, monkeypatch):
+    """Both sides of UNA_CORRIENTE, each against two streams: the same kernels in the same order of sums, so equal."""
+    vistas = []
+
+    def espiar(m):
+        m.largos[0].register_forward_pre_hook(lambda c, a, kw: vistas.append(kw.get('una_corriente', False)),
+                                              with_kwargs=True)
+    got = _paso_pequeno(B, L, d, espiar)
+    monkeypatch.setattr(modelo, 'UNA_CORRIENTE', -1)
+    ref = _paso_pequeno(B, L, d, espiar)
+    assert vistas == [una, False]
+    for a, b in zip(got, ref):
+        assert torch.equal(a, b)
