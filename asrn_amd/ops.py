@@ -1418,7 +1418,10 @@ def incrustar(emb, x):
 def recortar_gradientes(params, maximo, perdida):
     """clip_grad_norm_(params, maximo) and the step's check in three launches (asrn_clip_gradients): the gradients are
     scaled in place; returns (their norm, 1.0 when the loss or the norm is not finite else 0.0) as device scalars.
-    None when a gradient or the loss is not a contiguous fp32 tensor on one GPU."""
+    None when a gradient or the loss is not a contiguous fp32 tensor on one GPU, or the limit not a number from 0 on (a
+    device tensor, a negative limit): clip_grad_norm_ takes those."""
+    if not isinstance(maximo, (int, float)) or not maximo >= 0:
+        return None
     gs = [p.grad for p in params if p.grad is not None]
     if not gs or not perdida.is_cuda or not all(
             g.device == perdida.device and g.dtype == torch.float32 and g.layout == torch.strided and g.is_contiguous()

@@ -4,7 +4,8 @@ no limit, and non-finite gradients and losses. fp32 sums of up to 8,192 squares:
 import pytest
 import torch
 
-from asrn_amd import ops
+import asrn_amd
+from asrn_amd import ops, synth
 
 pytestmark = pytest.mark.gpu
 
@@ -50,3 +51,24 @@ def test_other_types_are_left_to_torch():
     p = torch.nn.Parameter(torch.zeros(4, device='cuda', dtype=torch.float64))
     p.grad = torch.ones_like(p)
     assert ops.recortar_gradientes([p], 1.0, torch.tensor(1.0, device='cuda')) is None
+
+
+@pytest.mark.parametrize('maximo', [-1.0, float('nan'), 'tensor'])
+def test_other_limits_are_left_to_torch(maximo):
+    a = _params([5], 1.0, 3)
+    limite = torch.tensor(0.5, device='cuda') if maximo == 'tensor' else maximo
+    antes = [p.grad.clone() for p in a]
+    assert ops.recortar_gradientes(a, limite, torch.tensor(1.0, device='cuda')) is None
+    assert all(torch.equal(p.grad, g) for p, g in zip(a, antes))
+
+
+def test_graphed_step_takes_a_negative_limit():
+    """PasoGrafado with a negative limit: the captured clipping is clip_grad_norm_'s, the gradient turned round."""
+    m = asrn_amd.crear_modelo(97, d=64, n_capas=2, semilla=1).cuda().train()
+    opt = asrn_amd.crear_optimizador(m, lr=1e-3, capturable=True)
+    paso = asrn_amd.PasoGrafado(m, opt, 2, 64, precision='fp32', recorte=-0.5)
+    w = synth.tokens(2, 65, 97, seed=1).cuda()
+    for _ in range(5):
+        _, norma, salto = paso(w[:, :-1].contiguous(), w[:, 1:].contiguous(), lr=0.0)
+    total = torch.stack([p.grad.norm() for p in paso.params]).norm()
+    assert salto.item() == 0 and norma.item() > 0 and abs(total.item() - 0.5) <= 1e-4 * 0.5
