@@ -47,3 +47,29 @@ def test_rates_from_logarithms(B, L, n):
         res.append((h, r) + torch.autograd.grad((h * wh).sum() + (r * wr).sum(), (lk, lr)))
     for a, b in zip(*res):
         torch.testing.assert_close(a, b, rtol=1e-5, atol=1e-5 * b.abs().max().item())
+
+
+@pytest.mark.parametrize('B,L,n', [(700, 3, 4), (53, 40, 1), (3, 60, 254), (2, 60, 255), (2, 60, 300)])
+def test_rates_gradients_over_batches_and_groups(B, L, n):
+    """The rates' gradients: batches of less and more than a run of rows a lane, and rates around the workgroup's 256,
+    against the two functions whose sums over the batch torch forms. fp32 sums of B rows: 2^-24 B of their magnitudes."""
+    g = torch.Generator(device='cuda').manual_seed(B + n)
+    order = torch.rand(B, n, L, generator=g, device='cuda').argsort(-1)
+    rank_k = order.argsort(-1).int()
+    order = order.int()
+    rep = (torch.rand(B, n, L, generator=g, device='cuda') < 0.5).to(torch.uint8)
+    rep[..., 0] = 0
+    vistos = torch.rand(B, L, n, generator=g, device='cuda')
+    beta = torch.rand(B, L, generator=g, device='cuda', dtype=torch.float64)
+    Bt, la = beta.cumsum(1), -torch.rand(B, L, generator=g, device='cuda')
+    k = torch.rand(n, generator=g, device='cuda').requires_grad_()
+    kr = torch.tensor([0.3], device='cuda', requires_grad=True)
+    wh, wr = torch.randn(B, L, n, generator=g, device='cuda'), torch.randn(B, L, generator=g, device='cuda')
+    h, r = ops.Repeticion.apply(Bt, la, k, beta, kr, order, rep, rank_k, vistos)
+    got = torch.autograd.grad((h * wh).sum() + (r * wr).sum(), (k, kr))
+    h2, r2 = ops.Hawkes.apply(Bt, la, k, order, rep, rank_k), ops.Streak.apply(beta, kr, vistos)
+    assert torch.equal(h, h2) and torch.equal(r, r2)
+    ref = torch.autograd.grad((h2 * wh).sum() + (r2 * wr).sum(), (k, kr))
+    for a, b in zip(got, ref):
+        mag = B ** 0.5 * b.norm().item() / b.numel() ** 0.5 + b.abs().max().item()
+        assert (a - b).abs().max().item() <= 2.0 ** -24 * B * mag
