@@ -28,9 +28,10 @@ MODOS_CHECKPOINT = ('no', 'asrn', 'todo')
 # without branches replays with its launches back to back, one with a branch pays for them one by one, and below this
 # the launches cost more than the layers' two branches gain by running side by side (us a step, two streams / one: 512
 # tokens at d 64 690 / 599, 4096 at d 64 785 / 723, 4096 at d 256 1365 / 1324, 4096 at d 512 2588 / 2603); an eager step is bound
-# by the host and saves the second stream's events (4096 at d 64 3927 / 3606, at d 256 3644 / 3346). Only where the
-# embedding's gradient is the library's too (ops.incrustar_ok): torch's for longer batches, replayed back to back in a graph
-# without branches, ended in an illegal access in its own partition kernel (16 x 1024 tokens, d 64), cause not known.
+# by the host and saves the second stream's events (4096 at d 64 3927 / 3606, at d 256 3644 / 3346). Not where
+# torch sorts the tokens for the embedding's gradient (past ops.FICHAS_EN_FILA of them, and not ops.incrustar_ok): replayed back
+# to back in a graph without branches that sort ended in an illegal access in its own partition kernel (16 x 1024 tokens, d
+# 64), cause not known.
 UNA_CORRIENTE = 1 << 20
 
 
@@ -223,7 +224,8 @@ class ModeloASRN(nn.Module):
         ck_capa = recalcular and self.checkpoint != 'no'
         # the n-gram sort depends on the token ids only: one for every ASRN layer
         ng = ngramas(x, self.largos[0]) if len(self.largos) and x.is_cuda else None
-        una = recalcular and E.numel() <= UNA_CORRIENTE and ops.incrustar_ok(self.emb, x)
+        una = (recalcular and E.numel() <= UNA_CORRIENTE
+               and (x.numel() <= ops.FICHAS_EN_FILA or ops.incrustar_ok(self.emb, x)))
         capas = iter(self.largos)
         h = E
         for i, bloque in enumerate(self.bloques):

@@ -1374,6 +1374,14 @@ def cross_entropy(logits, target, ignore_index=-100, reduction='mean'):
 # ---------------------------------------------------------------------------------------------------------------------
 
 FICHAS_INCRUSTAR = 4096      # most tokens asrn_embedding_bwd takes; past them torch's sort-based backward runs
+FICHAS_EN_FILA = 3072        # tokens torch's backward walks one by one; past them it sorts them
+# asrn_embedding_bwd reads every id once per 16 rows and 64 columns of the weight, 1.8 us per 2^20 of its elements, torch's
+# fill 0.6 and its walk 45 ns a token: the first one up to this many elements a token (us, own / torch: 64 tokens at d 64, V
+# 32768 7 / 7, at d 768, V 8000 15 / 10; 512 tokens at d 1536, V 8000 31 / 41, at d 768, V 32768 49 / 47; 2048 at d 1536,
+# V 32768 107 / 151), and past FICHAS_EN_FILA up to this many in all (4096 tokens at d 1536, V 8000 60 / 91, at d 256, V 131072
+# 100 / 78)
+PESO_POR_FICHA = 1 << 15
+PESO_ORDENADO = 3 << 23
 
 
 class Incrustar(torch.autograd.Function):
@@ -1397,8 +1405,10 @@ class Incrustar(torch.autograd.Function):
 
 def incrustar_ok(emb, x):
     """Whether incrustar(emb, x) runs asrn_embedding_bwd: a plain fp32 nn.Embedding in training on the GPU, whose call
-    is its class's forward and no hooks, up to FICHAS_INCRUSTAR int64 tokens."""
+    is its class's forward and no hooks, up to FICHAS_INCRUSTAR int64 tokens, and the faster one for its size."""
     w = emb.weight
+    if w.numel() > (x.numel() * PESO_POR_FICHA if x.numel() <= FICHAS_EN_FILA else PESO_ORDENADO):
+        return False
     return (w.is_cuda and x.device == w.device and x.dtype == torch.int64 and w.dtype == torch.float32 and w.requires_grad
             and torch.is_grad_enabled() and 1 <= x.numel() <= FICHAS_INCRUSTAR and type(emb) is torch.nn.Embedding
             and emb.padding_idx is None and emb.max_norm is None and not emb.scale_grad_by_freq and not emb.sparse

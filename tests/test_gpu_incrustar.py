@@ -50,3 +50,19 @@ def test_global_hooks_and_a_replaced_forward_run():
         assert vistos == [emb]
     emb.forward = lambda x: 2 * torch.nn.functional.embedding(x, emb.weight)
     assert torch.equal(ops.incrustar(emb, x), 2 * emb.weight[x])
+
+
+@pytest.mark.parametrize('n,V,d,propio', [(64, 32768, 64, True), (64, 32769, 64, False), (3072, 49152, 64, True),
+                                          (3073, 393216, 64, True), (3073, 393217, 64, False), (4097, 8, 8, False)])
+def test_size_rule(n, V, d, propio):
+    """Both sides of the rule's lines, on the gradient that the chosen side gives."""
+    emb = torch.nn.Embedding(V, d).cuda()
+    g = torch.Generator(device='cuda').manual_seed(n)
+    x = torch.randint(0, V, (n,), generator=g, device='cuda')
+    gy = torch.randn(n, d, generator=g, device='cuda')
+    y = ops.incrustar(emb, x)
+    assert ops.incrustar_ok(emb, x) == propio == ('Incrustar' in type(y.grad_fn).__name__)
+    dw, = torch.autograd.grad(y, emb.weight, gy)
+    ref = torch.zeros(V, d, dtype=torch.float64, device='cuda').index_add_(0, x, gy.double())
+    mag = torch.zeros_like(ref).index_add_(0, x, gy.double().abs())
+    assert bool(((dw.double() - ref).abs() <= 2.0 ** -24 * n ** 0.5 * mag + 1e-30).all())
