@@ -28,10 +28,8 @@ MODOS_CHECKPOINT = ('no', 'asrn', 'todo')
 # without branches replays with its launches back to back, one with a branch pays for them one by one, and below this
 # the launches cost more than the layers' two branches gain by running side by side (us a step, two streams / one: 512
 # tokens at d 64 690 / 599, 4096 at d 64 785 / 723, 4096 at d 256 1365 / 1324, 4096 at d 512 2588 / 2603); an eager step is bound
-# by the host and saves the second stream's events (4096 at d 64 3927 / 3606, at d 256 3644 / 3346). Not where
-# torch sorts the tokens for the embedding's gradient (past ops.FICHAS_EN_FILA of them, and not ops.incrustar_ok): replayed back
-# to back in a graph without branches that sort ended in an illegal access in its own partition kernel (16 x 1024 tokens, d
-# 64), cause not known.
+# by the host and saves the second stream's events (4096 at d 64 3927 / 3606, at d 256 3644 / 3346). Which steps else:
+# ModeloASRN._una_corriente.
 UNA_CORRIENTE = 1 << 20
 
 
@@ -215,6 +213,17 @@ class ModeloASRN(nn.Module):
     def checkpoint(self, valor):
         self._checkpoint = modo_checkpoint(valor)
 
+    def _una_corriente(self, E, x):
+        """Whether a training step over x keeps its ASRN layers on one stream. Captured, it is then a graph without
+        branches, and there a memset that a torch op records is not safe in replays queued back to back: the sort in
+        torch's embedding gradient, which clears its state that way, ended in an illegal access in its partition kernel
+        (16 x 1024 tokens, d 64). So only steps without such ops: torch does not sort the tokens (up to
+        ops.FICHAS_EN_FILA of them, or the library's gradient), the blocks are the fused 'conv' ones ('memoria' sums its
+        parameters' gradients in torch, with a cleared counter) and d is one the fused kernels take."""
+        return (E.numel() <= UNA_CORRIENTE and E.shape[-1] <= 1024
+                and (x.numel() <= ops.FICHAS_EN_FILA or ops.incrustar_ok(self.emb, x))
+                and all(type(b) is BloqueLocal and b.mezcla == 'conv' for b in self.bloques))
+
     def estado(self, x):
         """The last block's output, before ln_f and the head: (B, L, d)."""
         revisar_precision(self)
@@ -224,8 +233,7 @@ class ModeloASRN(nn.Module):
         ck_capa = recalcular and self.checkpoint != 'no'
         # the n-gram sort depends on the token ids only: one for every ASRN layer
         ng = ngramas(x, self.largos[0]) if len(self.largos) and x.is_cuda else None
-        una = (recalcular and E.numel() <= UNA_CORRIENTE
-               and (x.numel() <= ops.FICHAS_EN_FILA or ops.incrustar_ok(self.emb, x)))
+        una = recalcular and self._una_corriente(E, x)
         capas = iter(self.largos)
         h = E
         for i, bloque in enumerate(self.bloques):

@@ -388,12 +388,36 @@ class _Envoltura(torch.nn.Module):
 
 
 def _paso_pequeno(B, L, d, cambio=None):
-    m = asrn_amd.crear_modelo(97, d=d, n_capas=2, semilla=3, **REDUCIDA).to(DEV).train()
+    m = asrn_amd.crear_modelo(97, d, n_capas=2, semilla=3, **REDUCIDA).to(DEV).train()
     if cambio:
         cambio(m)
     w = synth.tokens(B, L + 1, 97, seed=4).to(DEV)
     perdida = m.perdida(w[:, :-1].contiguous(), w[:, 1:].contiguous())
     return [perdida.detach(), *torch.autograd.grad(perdida, list(m.parameters()))]
+
+
+@pytest.mark.parametrize('kw,B,L', [(dict(d=64, mezcla='memoria'), 4, 128), (dict(d=1028), 1, 100)])
+def test_steps_with_torch_sums_keep_two_streams(kw, B, L):
+    """Captured steps that hold torch's multi-workgroup sums (memset nodes): branches as before, and every replay's
+    gradients equal an ordinary step's."""
+    m = asrn_amd.crear_modelo(97, n_capas=2, semilla=3, **kw, **REDUCIDA).to(DEV).train()
+    m2 = copy.deepcopy(m)
+    vistas = []
+    m.largos[0].register_forward_pre_hook(lambda c, a, kw: vistas.append(kw.get('una_corriente', False)), with_kwargs=True)
+    opt = asrn_amd.crear_optimizador(m, lr=0.0, capturable=True)
+    paso = asrn_amd.PasoGrafado(m, opt, B, L, precision='fp32', calentar=2)
+    w = synth.tokens(3 * B, L + 1, 97, seed=4).to(DEV)
+    for i in range(6):
+        x, y = w[B * (i % 3):B * (i % 3 + 1), :-1].contiguous(), w[B * (i % 3):B * (i % 3 + 1), 1:].contiguous()
+        paso(x, y, lr=0.0)
+        torch.cuda.synchronize()
+        got = [p.grad.clone() for p in m.parameters()]
+        ref = torch.autograd.grad(m2.perdida(x, y), list(m2.parameters()))
+        norma = torch.stack([g.norm() for g in ref]).norm().item()
+        factor = min(1.0, 1.0 / (norma + 1e-6))
+        for (n, p), a, b in zip(m.named_parameters(), got, ref):
+            assert (a - factor * b).norm().item() <= 1e-5 * (factor * b).norm().item() + 1e-7 * min(norma, 1.0), (i, n)
+    assert not any(vistas)
 
 
 @pytest.mark.parametrize('modo', ['envoltura', 'forward', 'subclase'])
