@@ -1567,9 +1567,9 @@ class SumaGeluNorma(torch.autograd.Function):
 
 def suma_gelu_norma(ln, h, c, dtype):
     """(LayerNorm ln of h + gelu(c) in `dtype`, h + gelu(c)): fused where norma_residual's is and h is fp32, c fp32 or
-    bf16; else the separate ops."""
+    bf16, both on the 16-byte boundary that the kernel reads from; else the separate ops, whose sum lies on one."""
     d = h.shape[-1]
-    if (h.is_cuda and h.dtype == torch.float32 and c.dtype in (torch.float32, torch.bfloat16) and c.shape == h.shape
+    if (h.is_cuda and h.dtype == torch.float32 and not (h.data_ptr() | c.data_ptr()) % 16 and c.dtype in (torch.float32, torch.bfloat16) and c.shape == h.shape
             and dtype in (torch.float32, torch.bfloat16) and d % 4 == 0 and d <= 1024 and ln.elementwise_affine
             and ln.bias is not None and tuple(ln.normalized_shape) == (d,)):
         return SumaGeluNorma.apply(h, c, ln.weight, ln.bias, ln.eps, dtype)

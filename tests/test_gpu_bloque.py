@@ -35,3 +35,19 @@ def test_matches_torch(rows, d, dc, dy):
     for a, b in zip(got, ref):
         e = 2.0 ** -7 if a.dtype == torch.bfloat16 or dc == torch.bfloat16 else 5e-6
         assert ((a - b).float().norm() / b.float().norm().clamp(min=1e-20)).item() <= e
+
+
+@pytest.mark.parametrize('cual', ['h', 'c'])
+def test_rows_off_a_16_byte_boundary(cual):
+    """A residual or a convolution output that is a view into a flat buffer: the separate ops take it."""
+    g = torch.Generator(device='cuda').manual_seed(5)
+    ln = torch.nn.LayerNorm(64).cuda()
+    t = {k: torch.randn(10 * 64 + 1, generator=g, device='cuda')[1 if k == cual else 0:][:640].view(10, 64) for k in 'hc'}
+    h, c = t['h'].requires_grad_(), t['c'].requires_grad_()
+    y, x = ops.suma_gelu_norma(ln, h, c, torch.float32)
+    ref = h + F.gelu(c)
+    torch.testing.assert_close(x, ref, rtol=1e-6, atol=1e-6)
+    torch.testing.assert_close(y, ln(ref), rtol=1e-5, atol=1e-5)
+    got, exp = (torch.autograd.grad(o.sum() + (o * o).sum(), (h, c), retain_graph=True) for o in (x, ref))
+    for a, b in zip(got, exp):
+        torch.testing.assert_close(a, b, rtol=1e-5, atol=1e-5)
