@@ -7,7 +7,10 @@
 // below fp32's own rounding of each product, and fewer roundings of the running sum (one per 16 terms and product
 // order). Measured against 64 bits over the declared sizes the results are no further off than the library's fp32
 // products. A value that is not finite, or rounds to infinity in bf16, turns its products into NaN here; results that
-// come out not finite are formed again as plain fp32 sums (redo), so infinities and NaN are those of an fp32 product.
+// come out not finite are formed again as plain fp32 sums, so infinities and NaN are those of an fp32 product. A wave
+// forms its rows' 32 by 32 blocks that hold such results again, the operands through LDS unsplit: a product that is all
+// NaN takes 4 to 5 times a finite one's time (768 x 3072 over 12000 tokens with one NaN token 338 us finite, 1.5 ms; one
+// result after the other by its thread 62 ms), so a training step that is to be skipped stays a step.
 // bf16 operands (TN only, the weight gradients): the products as they are, summed in fp32.
 //
 // The matrix cores drop the low bits of a sum towards minus infinity (measured: 256 terms leave results low by 1.5e-8
@@ -171,6 +174,16 @@ struct Operand {
       }
     }
   }
+  // F32: the units' values as they are, row r of step column k at lds[k * R + r]
+  __device__ __forceinline__ void store_raw(float* lds, int tid) const {
+#pragma unroll
+    for (int i = 0; i < U; ++i) {
+      int c, r;
+      where(tid, i, c, r);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) lds[(8 * c + j) * R + r] = f[i][j];
+    }
+  }
   // adds this step's values to the thread's U column sums (T)
   __device__ __forceinline__ void column_sums(float (&s)[U]) const {
 #pragma unroll
@@ -185,13 +198,6 @@ struct Operand {
     }
   }
 };
-
-template <bool T, bool F32>
-__device__ __forceinline__ float element(const void* X, int64_t ld, int r, int k) {
-  const int64_t at = T ? (int64_t)k * ld + r : (int64_t)r * ld + k;
-  if constexpr (F32) return static_cast<const float*>(X)[at];
-  else return __uint_as_float((uint32_t)static_cast<const uint16_t*>(X)[at] << 16);
-}
 
 // k per step: 64 for bf16; for fp32 32, or 64 in the smallest tile, whose few steps wait for their loads
 template <int BM, int BN, bool F32>
@@ -303,18 +309,64 @@ __global__ __launch_bounds__(kGemmThr, 2) void k_gemm(Gemm g) {
       }
     }
   if constexpr (F32) {
-    while (bad) {                                 // plain fp32 sums, one element at a time (infinities and NaN only)
-      const int x = __ffsll((unsigned long long)bad) - 1;
-      bad &= bad - 1;
-      const int e = x & 15, ij = x >> 4, i = ij / NI, j = ij % NI;
-      const int m = m0 + wm + 32 * i + 8 * (e >> 2) + 4 * lc + (e & 3), n = n0 + wn + 32 * j + lr;
-      float v = 0.f;
-      for (int k = ka; k < kb; ++k)
-        v = fmaf(element<TA, F32>(g.A, g.lda, m, k), element<TB, F32>(g.B, g.ldb, n, k), v);
-      float* o = out + (int64_t)m * ldo + n;
-      if (last && g.bias) v += g.bias[n];
-      if (last && g.accumulate) v += *o;
-      *o = v;
+    if (__syncthreads_or(bad != 0)) {             // uniform: once more as plain fp32 sums, k in order
+      static_assert(BK * (BM + BN) * 4 <= sizeof(lds), "the values of a step fit where their parts did");
+      float* ra = reinterpret_cast<float*>(lds);
+      float* rb = ra + BK * BM;
+#pragma unroll
+      for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int j = 0; j < NI; ++j)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+      bool some[MI];                              // whether the wave has such results in its rows' i-th 32 (uniform)
+#pragma unroll
+      for (int i = 0; i < MI; ++i) some[i] = __any((bad >> (i * NI * 16) & ((1ull << NI * 16) - 1)) != 0);
+      load(ka);
+      for (int k = ka; k < kb; k += BK) {
+        __syncthreads();
+        a.store_raw(ra, tid);
+        b.store_raw(rb, tid);
+        __syncthreads();
+        if (k + BK < kb) load(k + BK);
+#pragma unroll 2
+        for (int kk = 0; kk < BK; ++kk) {         // past kb both operands are 0
+          float y[NI];
+#pragma unroll
+          for (int j = 0; j < NI; ++j) y[j] = rb[kk * BN + wn + 32 * j + lr];
+#pragma unroll
+          for (int i = 0; i < MI; ++i) {
+            if (!some[i]) continue;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+              const float4 x = *reinterpret_cast<const float4*>(ra + kk * BM + wm + 32 * i + 8 * q + 4 * lc);
+#pragma unroll
+              for (int j = 0; j < NI; ++j) {
+                acc[i][j][4 * q] = fmaf(x.x, y[j], acc[i][j][4 * q]);
+                acc[i][j][4 * q + 1] = fmaf(x.y, y[j], acc[i][j][4 * q + 1]);
+                acc[i][j][4 * q + 2] = fmaf(x.z, y[j], acc[i][j][4 * q + 2]);
+                acc[i][j][4 * q + 3] = fmaf(x.w, y[j], acc[i][j][4 * q + 3]);
+              }
+            }
+          }
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int j = 0; j < NI; ++j) {
+          const int n = n0 + wn + 32 * j + lr;
+          const float bias = last && g.bias && n < g.N ? g.bias[n] : 0.f;
+#pragma unroll
+          for (int e = 0; e < 16; ++e) {
+            if (!(bad >> ((i * NI + j) * 16 + e) & 1)) continue;     // inside the matrix, and not stored above
+            const int m = m0 + wm + 32 * i + 8 * (e >> 2) + 4 * lc + (e & 3);
+            float* o = out + (int64_t)m * ldo + n;
+            float v = acc[i][j][e] + bias;
+            if (last && g.accumulate) v += *o;
+            *o = v;
+          }
+        }
     }
   }
   if constexpr (TA) {

@@ -179,3 +179,28 @@ def test_no_input_features(dt):
     del poison
     gw, gb = torch.autograd.grad(lineal(x, w, b), (w, b), gy)
     assert gw.shape == w.shape and bool((gb == 700).all())
+
+
+@pytest.mark.parametrize('tile', [128 << 8 | 128, 64 << 8 | 64])
+@pytest.mark.parametrize('ta,tb', [(0, 1), (0, 0), (1, 0)])
+@pytest.mark.parametrize('splits', [1, 3])
+def test_tiles_with_infinities_and_nan(tile, ta, tb, splits):
+    """Tiles formed again as plain fp32 sums, in every layout, with a ragged last step: rows with a NaN, infinities of
+    both signs and a value that rounds to infinity in bf16 (against operands small enough for a finite result)."""
+    M, N, K = 260, 136, 700
+    g = torch.Generator(device='cuda').manual_seed(7)
+    a, b = torch.randn(M, K, generator=g, device='cuda'), torch.randn(N, K, generator=g, device='cuda')
+    b[:, 690] *= 1e-37
+    a[3, 690], a[130, 1], a[131, 1], a[259, 690] = 3.4e38, float('nan'), float('inf'), -3.4e38
+    a[200, 5], a[200, 6] = float('inf'), float('-inf')
+    exact = a.double() @ b.double().t()
+    out = torch.empty(M, N, device='cuda')
+    bias = torch.randn(N, generator=g, device='cuda')
+    _llamar(a.t().contiguous() if ta else a, ta, b if tb else b.t().contiguous(), tb, M, N, K, out, tile, splits, bias=bias)
+    exact = exact + bias.double()
+    fin = torch.isfinite(exact)
+    assert torch.equal(torch.isnan(out), torch.isnan(exact)) and torch.equal(out[torch.isinf(exact)].double(),
+                                                                               exact[torch.isinf(exact)])
+    # a row's plain sum of K terms: 2^-24 sqrt(K) of the terms' norm, as the others'
+    escala = (a.double().square() @ b.double().square().t()).sqrt() + bias.abs().double()
+    assert bool(((out.double() - exact).abs()[fin] <= 2.0 ** -24 * 4 * (2 + K ** 0.5) * escala[fin]).all())
