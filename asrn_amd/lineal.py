@@ -5,8 +5,8 @@ For y = x W^T + b over N tokens, the weight gradient dW = dY^T X reduces over al
 shape) into a small (out, in) matrix. As one GEMM it has only (out / tile) x (in / tile) output tiles to spread over
 256 CUs. asrn_gemm cuts the token axis into slabs whose partial products are added in order, and sums the bias
 gradient (dY's columns) from the values it loads anyway. fp32 products run there on the bf16 matrix cores, each operand
-split into three bf16 parts: fp32's error at more than fp32's matrix rate. Where hipBLASLt is faster (below), it is
-called as before: the weight gradient as one batched product over slabs of tokens.
+split into three bf16 parts: fp32's error (for operands from 2^-110 on) at more than fp32's matrix rate. Where hipBLASLt
+is faster (below), it is called as before: the weight gradient as one batched product over slabs of tokens.
 Under autocast the operands are cast as autocast casts F.linear's, and the products run in that dtype.
 
 On the GPU, the sums (the slab partials, and the bias gradients' column sums) run in the library's asrn_column_sums
@@ -78,23 +78,22 @@ def _apto(t):
             and t.data_ptr() % (4 * t.element_size()) == 0)
 
 
-def gemm(a, ta, b, tb, out=None, sesgo=None, sumar=False, columnas=False):
-    """op(a) op(b) (+ sesgo) in fp32 on asrn_gemm, op the transpose where ta, tb; sumar: added into out. columnas (ta):
-    returns (product, the sums of a's columns). Shapes that do not chain are refused here: the kernels see leading
-    dimensions only and would read whatever lies there."""
+def gemm(a, ta, b, tb, sesgo=None, columnas=False):
+    """op(a) op(b) (+ sesgo) in fp32 on asrn_gemm, op the transpose where ta, tb. columnas (ta): returns (product, the
+    sums of a's columns). Shapes that do not chain are refused here: the kernels see leading dimensions only and would
+    read whatever lies there."""
     M, K = (a.shape[1], a.shape[0]) if ta else a.shape
     Kb, N = (b.shape[1], b.shape[0]) if tb else b.shape
     if K != Kb or (sesgo is not None and tuple(sesgo.shape) != (N,)):
         raise ValueError(f'gemm: shapes {tuple(a.shape)}{" transposed" if ta else ""}, {tuple(b.shape)}'
                          f'{" transposed" if tb else ""} and bias {None if sesgo is None else tuple(sesgo.shape)} do not chain')
     bf = int(a.dtype == torch.bfloat16)
-    if out is None:
-        out = torch.empty((M, N), dtype=torch.float32, device=a.device)
+    out = torch.empty((M, N), dtype=torch.float32, device=a.device)
     cols = torch.empty((M,), dtype=torch.float32, device=a.device) if columnas else None
     wsb = _lib.query('asrn_gemm_workspace', M, N, K, bf, int(columnas), 0, 0)
     ws = torch.empty((wsb,), dtype=torch.uint8, device=a.device) if wsb > 0 else None
     _lib.call('asrn_gemm', _lib.ptr(a), a.stride(0), int(ta), _lib.ptr(b), b.stride(0), int(tb), bf, _lib.ptr(out),
-              out.stride(0), M, N, K, _lib.ptr(sesgo), int(sumar), _lib.ptr(cols), 0, 0, _lib.ptr(ws), wsb,
+              out.stride(0), M, N, K, _lib.ptr(sesgo), 0, _lib.ptr(cols), 0, 0, _lib.ptr(ws), wsb,
               _lib.stream_of(a.device))
     return (out, cols) if columnas else out
 
