@@ -1,16 +1,18 @@
 // Dense products on the bf16 matrix cores with fp32 results: C (M, N) = op(A) op(B) (+ C) (+ bias).
 //
-// fp32 operands (F32): CDNA4's fp32 matrix rate is 157 TFLOP/s, its bf16 rate 16 times that. An fp32 value is exactly
-// the sum of three bf16 values (24 significand bits in three parts of 8, each part the previous remainder rounded to
-// nearest), so a product x y is the sum of nine bf16 products, exact in the fp32 accumulator's input. The three
-// smallest (second x third and below, at most 2^-25 of x y) are left out: six bf16 products per fp32 one, an error
+// fp32 operands (F32): CDNA4's fp32 matrix rate is 157 TFLOP/s, its bf16 rate 16 times that. An fp32 value from 2^-110
+// on is exactly the sum of three bf16 values (24 significand bits in three parts of 8, each part the previous remainder
+// rounded to nearest), so a product x y is the sum of nine bf16 products, exact in the fp32 accumulator's input. The
+// three smallest (second x third and below, at most 2^-25 of x y) are left out: six bf16 products per fp32 one, an error
 // below fp32's own rounding of each product, and fewer roundings of the running sum (one per 16 terms and product
-// order). Measured against 64 bits over the declared sizes the results are no further off than the library's fp32
-// products. A value that is not finite, or rounds to infinity in bf16, turns its products into NaN here; results that
-// come out not finite are formed again as plain fp32 sums, so infinities and NaN are those of an fp32 product. A wave
-// forms its rows' 32 by 32 blocks that hold such results again, the operands through LDS unsplit: a product that is all
-// NaN takes 4 to 5 times a finite one's time (768 x 3072 over 12000 tokens with one NaN token 338 us finite, 1.5 ms; one
-// result after the other by its thread 62 ms), so a training step that is to be skipped stays a step.
+// order). Measured against 64 bits (256 to 65536 terms, centred and positive operands) the products are half as far off as
+// the library's fp32 ones or less. Below 2^-110 a remainder may lie under bf16's smallest subnormal, and the value enters
+// rounded to a multiple of 2^-133: products of values around 1e-35 are off by 2.7e-6, around 1e-38 by 2.7e-3.
+// A value that is not finite, or rounds to infinity in bf16, turns its products into NaN here; results that come out not
+// finite are formed again as plain fp32 sums, so infinities and NaN are those of an fp32 product. A wave forms its rows'
+// 32 by 32 blocks that hold such results again, the operands through LDS unsplit: a product that is all NaN takes 4 to 5
+// times a finite one's time (768 x 3072 over 12000 tokens with one NaN token 338 us finite, 1.5 ms; one result after the
+// other by its thread 62 ms), so a training step that is to be skipped stays a step.
 // bf16 operands (TN only, the weight gradients): the products as they are, summed in fp32.
 //
 // The matrix cores drop the low bits of a sum towards minus infinity (measured: 256 terms leave results low by 1.5e-8
@@ -25,8 +27,8 @@
 // A workgroup of 4 waves forms a BM x BN tile, each wave a quarter of it from 32x32x16 MFMA tiles. Operands are loaded
 // into registers one step ahead, split there and stored to LDS in units of 8 consecutive k of one row, the operand an
 // MFMA lane takes; an operand stored with its rows contiguous (TA, TB) is transposed on the way, 8 k-rows per thread,
-// which costs nothing in fp32 and one permute per pair in bf16. Two workgroups share a CU (50-57 KB of LDS, 256
-// registers a wave): one's loads, splits and barriers run under the other's MFMA.
+// which costs nothing in fp32 and one permute per pair in bf16. Three workgroups share a CU in fp32 (49,920 bytes of LDS
+// and 112 to 164 registers a wave): one's loads, splits and barriers run under the others' MFMA.
 // Products with few tiles (weight gradients: K is the token axis) are cut along K: partial products in a workspace,
 // summed in order by a second launch. No atomics: the result is a function of the sizes alone.
 // The weight gradient's bias gradient, the column sums of A (TA), is summed from the values a tile loads anyway.
@@ -615,8 +617,25 @@ __global__ __launch_bounds__(kGemmThr) void k_gemm_tail(Gemm g, int bm, int bn) 
 
 struct Plan { int bm, bn, splits, kper, tail, tsplits, tkper; };
 
-constexpr int kSlots = 512;     // workgroups that run at once, 2 a CU
+constexpr int kSlots = 512;     // workgroups that a plan counts on running at once, 2 a CU
 
+// The tile and the slabs of K by the sizes. Each line with both sides measured (us, without the column sums):
+// 128 x 128 in fp32 from 448 of them on: a smaller one splits its operands' values more often, but fewer large ones leave
+//   slots idle. 64 / 128: 4096 x 768 x 768 (192 tiles) 45 / 49, 4096 x 1536 x 256 (384) 28.5 / 29.3, 7168 x 1024 x 256
+//   (448) 34 / 30, 9600 x 768 x 768 (450) 87 / 68; at 384 to 447 tiles the long K already gain (8192 x 768 x 768 73 / 65).
+//   And for weights of 768 x 768 on over 2,048 and more, whose slabs fill the slots: 768 x 768 over 1536 28 / 31, over 2048
+//   33 / 32, over 4096 54 / 44, over 16384 179 / 119; just below that size 704 x 768 over 8192 92 / 69.
+// 256 x 256 in bf16 from 2^20 elements on where a workgroup has steps enough: 9.6e9 multiply-adds, or twice the elements.
+//   128 / 256: 1024 x 1024 over 8192 (8.6e9) 47 / 49, 768 x 1536 over 8192 (9.7e9) 52 / 52, over 10000 58 / 57, over 16384
+//   80 / 72; 768 x 3072 over 4096 58 / 58, over 8192 89 / 76.
+// The slabs fill the slots once (256 of the 256 x 256 tiles, one a CU): 768 x 3072 over 12000 (144 tiles) in 2, 3, 4 slabs
+//   460 / 350 / 411; 768 x 1536 over 12000 (72) in 4, 7, 14 236 / 172 / 198. A slab holds at least 64 of K, and 256 past
+//   K = 4096, for the sum over the slabs: 64 x 64 over 4096 in 32, 64 10.1 / 8.6; 128 x 128 over 16384 in 64, 128 15.6 /
+//   16.3, 256 x 256 over 8192 in 32, 64 20 / 23, though 64 x 64 over 8192 in 32, 64 13.4 / 10.3.
+// From 128 tiles on a K of up to 1,024 stays whole: 768 x 768 x 512 in 1, 3 slabs 15 / 16, 2048 x 512 x 1024 26 / 31,
+//   2304 x 256 x 768 20 / 19; at 128 to 144 tiles and the longest K it would gain (1024 x 512 x 1000 in 1, 4 25 / 19).
+// 64 x 128 and 128 x 64 are the caller's to ask for: between the two square ones nearly everywhere (768 x 768 over 4096 54 /
+//   48 / 49 / 44), ahead of both where those are about equal (4096 x 768 x 768 39 against 45 and 49).
 static Plan plan_of(int64_t M, int64_t N, int64_t K, bool f32, int tile, int splits) {
   Plan p;
   if (tile) {

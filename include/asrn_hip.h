@@ -202,8 +202,9 @@ int asrn_column_sums(const void* x, int32_t bf16, int64_t rows, int64_t cols, in
  * No counterpart in the reference's FFI: the products of its nn.Linear projections and their gradients
  * (asrn/nucleo.py:591-630, 969-1014), which it leaves to the framework's BLAS. C (M, N) fp32 = op(A) op(B) (+ C with
  * accumulate) (+ bias (N)), row-major with leading dimensions lda, ldb, ldc. bf16 = 0: fp32 operands, A (M, K) or, with
- * trans_a, stored (K, M); B (K, N) or, with trans_b, stored (N, K); not both. fp32 precision: each operand is split
- * into three bf16 parts whose products run on the matrix cores. bf16 != 0: bf16 operands, A stored (K, M) and B (K, N),
+ * trans_a, stored (K, M); B (K, N) or, with trans_b, stored (N, K); not both. Each operand is split into three
+ * bf16 parts whose products run on the matrix cores: fp32 precision for operands from 2^-110 on, smaller ones enter
+ * rounded to a multiple of 2^-133. bf16 != 0: bf16 operands, A stored (K, M) and B (K, N),
  * summed in fp32. colsum (M), with trans_a: also the sums of A's columns over K. N, M (trans_a) and K (an operand with
  * k contiguous) and the leading dimensions are multiples of 4, fp32 pointers 16-byte and bf16 ones 8-byte aligned.
  * tile: 0 (chosen by the sizes), rows << 8 | columns of 64 or 128, or for bf16 256 << 8 (256 x 256); splits: 0 (chosen)

@@ -215,3 +215,18 @@ def test_weight_gradients_errors_have_no_drift(M, N, K):
     exact = a.double().t() @ b.double()
     e = (gemm(a, True, b, False).double() - exact) / exact.square().mean().sqrt()
     assert abs(e.mean().item()) <= 5 * e.square().mean().sqrt().item() / (M * N) ** 0.5 + 1.5e-8
+
+
+@pytest.mark.parametrize('escala', [1e-30, 1e-33, 1e-35, 1e-37])
+def test_small_operands(escala):
+    """Operands down to fp32's smallest: exact in three parts from 2^-110 on, else rounded to a multiple of 2^-133, which
+    is off by 2^-134 at most; the bound adds that over K terms, at random, to the ordinary one."""
+    M, N, K = 200, 132, 260
+    g = torch.Generator(device='cuda').manual_seed(8)
+    a, b = escala * torch.randn(M, K, generator=g, device='cuda'), torch.randn(N, K, generator=g, device='cuda')
+    exact = a.double() @ b.double().t()
+    bound = 2.0 ** -24 * (2 + K ** 0.5) * exact.norm().item() + 2.0 ** -134 * (M * N * K) ** 0.5
+    for ta, tb, x, y in ((0, 1, a, b), (0, 0, a, b.t().contiguous()), (1, 0, a.t().contiguous(), b.t().contiguous())):
+        out = torch.empty(M, N, device='cuda')
+        _llamar(x, ta, y, tb, M, N, K, out, 0, 0)
+        assert (out.double() - exact).norm().item() <= bound
