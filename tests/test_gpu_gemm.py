@@ -6,7 +6,7 @@ import pytest
 import torch
 
 from asrn_amd import _lib, ops
-from asrn_amd.lineal import gemm, lineal, weight_grad
+from asrn_amd.lineal import _gradiente_ok, gemm, lineal, weight_grad
 
 pytestmark = pytest.mark.gpu
 TILES = [128 << 8 | 128, 64 << 8 | 128, 128 << 8 | 64, 64 << 8 | 64]
@@ -80,7 +80,7 @@ def test_infinities_and_nan_are_fp32s():
 @pytest.mark.parametrize('N,fin,fout', [(2049, 512, 516), (5003, 768, 128), (700, 64, 64), (700, 63, 65)])
 @pytest.mark.parametrize('dt', [torch.float32, torch.bfloat16])
 def test_lineal_matches_float64(N, fin, fout, dt):
-    """Sizes on both sides of every line of the dispatch, and sizes no own product takes, in a captured graph too."""
+    """Products past and below MIN_PRODUCTO, small weight gradients, and sizes no own product takes."""
     g = torch.Generator(device='cuda').manual_seed(N)
     x = torch.randn(N, fin, generator=g, device='cuda').to(dt).requires_grad_()
     w = (torch.randn(fout, fin, generator=g, device='cuda') / fin ** 0.5).to(dt).requires_grad_()
@@ -230,3 +230,74 @@ def test_small_operands(escala):
         out = torch.empty(M, N, device='cuda')
         _llamar(x, ta, y, tb, M, N, K, out, 0, 0)
         assert (out.double() - exact).norm().item() <= bound
+
+
+@pytest.mark.parametrize('dt,n,fout,fin,sesgo,propio', [
+    (torch.float32, 511, 96, 68, False, False), (torch.float32, 512, 96, 68, False, True),
+    (torch.float32, 4, 96, 68, True, True),
+    (torch.bfloat16, 5008, 256, 512, False, True), (torch.bfloat16, 5008, 260, 512, False, False),
+    (torch.bfloat16, 5003, 260, 512, False, True),
+    (torch.bfloat16, 2621, 1024, 1024, True, False), (torch.bfloat16, 2622, 1024, 1024, True, True),
+    (torch.bfloat16, 5242, 1024, 1024, False, False), (torch.bfloat16, 5243, 1024, 1024, False, True),
+    (torch.bfloat16, 9201, 1024, 1024, True, True), (torch.bfloat16, 6001, 2048, 1028, True, True)])
+def test_weight_gradients_on_both_sides_of_the_dispatch(dt, n, fout, fin, sesgo, propio):
+    """MIN_FICHAS in fp32; in bf16 MAX_PESO_16, the weights that slabs do not divide, FICHAS_PESO with and without the bias's
+    gradient, and sizes that the plan gives 256 x 256 tiles (the last two), through lineal."""
+    g = torch.Generator(device='cuda').manual_seed(n)
+    x = torch.randn(n, fin, generator=g, device='cuda').to(dt)
+    w = (torch.randn(fout, fin, generator=g, device='cuda') / fin ** 0.5).to(dt).requires_grad_()
+    b = torch.randn(fout, generator=g, device='cuda').to(dt).requires_grad_() if sesgo else None
+    gy = torch.randn(n, fout, generator=g, device='cuda').to(dt)
+    assert bool(_gradiente_ok(gy, x, sesgo)) == propio
+    got = torch.autograd.grad(lineal(x, w, b), (w, b) if sesgo else (w,), gy)
+    tol = 2.0 ** -24 * (4 + n ** 0.5) if dt == torch.float32 else 2.0 ** -8
+    d = lambda t: t.detach().double()
+    for o, e in zip(got, [d(gy).t() @ d(x), d(gy).sum(0)]):
+        assert _rel(o, e) <= tol
+
+
+@pytest.mark.parametrize('tb', [1, 0])
+def test_tail_tiles_of_64(tb):
+    """A second round of 64 x 64 tiles, ragged in rows, with an infinity in the last of them."""
+    M, N, K = 5005, 512, 256
+    g = torch.Generator(device='cuda').manual_seed(9)
+    a, bias = torch.randn(M, K, generator=g, device='cuda'), torch.randn(N, generator=g, device='cuda')
+    b = torch.randn(*((N, K) if tb else (K, N)), generator=g, device='cuda')
+    assert _lib.query('asrn_gemm_workspace', M, N, K, 0, 0, 0, 0) == (79 * 8 - 512) * 2 * 64 * 64 * 4
+    a[M - 1, 3] = float('inf')
+    exact = a.double() @ (b.double().t() if tb else b.double()) + bias
+    out = gemm(a, False, b, bool(tb), sesgo=bias)
+    assert torch.equal(out[M - 1], exact[M - 1].float())
+    assert _rel(out[:M - 1], exact[:M - 1]) <= 2.0 ** -24 * (3 + K ** 0.5)
+
+
+@pytest.mark.parametrize('dt,n,fin,fout', [(torch.float32, 5005, 256, 512), (torch.float32, 2600, 768, 260),
+                                           (torch.bfloat16, 2624, 1024, 1024)])
+def test_lineal_in_a_graph(dt, n, fin, fout):
+    """Forward and backward captured once (the tail's and the slabs' workspaces among the graph's buffers) and replayed
+    on new inputs, with other work between the replays: the ordinary call's bits each time."""
+    g = torch.Generator(device='cuda').manual_seed(n)
+    r = lambda *s: torch.randn(*s, generator=g, device='cuda').to(dt)
+    x, w, b, gy = r(n, fin).requires_grad_(), r(fout, fin).requires_grad_(), r(fout).requires_grad_(), r(n, fout)
+
+    def paso():
+        y = lineal(x, w, b)
+        return [y.detach(), *torch.autograd.grad(y, (x, w, b), gy)]
+    lado = torch.cuda.Stream()
+    lado.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(lado):
+        paso()
+    torch.cuda.current_stream().wait_stream(lado)
+    grafo = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(grafo):
+        out = paso()
+    for _ in range(4):
+        with torch.no_grad():
+            x.copy_(r(n, fin))
+        gy.copy_(r(n, fout))
+        for t in out:
+            t.fill_(-1.0)
+        grafo.replay()
+        torch.cuda.synchronize()
+        ref = paso()
+        assert all(torch.equal(u, v) for u, v in zip(out, ref))

@@ -9,7 +9,7 @@ from asrn_amd import _lib, ops
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize('V', [1, 9, 256, 257, 511, 512, 513, 1024, 2047, 2049, 4100])
+@pytest.mark.parametrize('V', [1, 9, 256, 257, 511, 512, 513, 1024, 2047, 2048, 2049, 4096, 4100, 8192, 8193])
 @pytest.mark.parametrize('dtype', [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize('por_vector', [1, 16])
 def test_lengths(V, dtype, por_vector):
