@@ -171,8 +171,8 @@ __global__ __launch_bounds__(THREADS) void k_ce_fwd(const void* logits, int64_t 
 // (8192 rows: 305 us for the whole loss either way).
 __global__ __launch_bounds__(kCeThreads) void k_ce_reduce(const float* loss, const int64_t* target, int64_t rows,
                                                           int64_t ignore, int mean, float* out, float* divisor) {
-  __shared__ double sums[kCeThreads];
-  __shared__ int counts[kCeThreads];               // rows < 2^31
+  __shared__ double sums[kCeWaves];
+  __shared__ int counts[kCeWaves];                 // rows < 2^31
   const int tid = threadIdx.x;
   double s = 0.0;
   int n = 0;
@@ -192,19 +192,23 @@ __global__ __launch_bounds__(kCeThreads) void k_ce_reduce(const float* loss, con
         n += t[u] != ignore;
       }
   }
-  sums[tid] = s;
-  counts[tid] = n;
-  __syncthreads();
-  for (int h = kCeThreads / 2; h > 0; h >>= 1) {
-    if (tid < h) {
-      sums[tid] += sums[tid + h];
-      counts[tid] += counts[tid + h];
-    }
-    __syncthreads();
+#pragma unroll
+  for (int m = kWave / 2; m >= 1; m >>= 1) {
+    s += __shfl_xor(s, m, kWave);
+    n += __shfl_xor(n, m, kWave);
   }
+  if ((tid & (kWave - 1)) == 0) {
+    sums[tid >> 6] = s;
+    counts[tid >> 6] = n;
+  }
+  __syncthreads();
   if (tid == 0) {
-    *out = (float)(mean ? sums[0] / counts[0] : sums[0]);
-    *divisor = mean ? (float)counts[0] : 1.f;
+    for (int w = 1; w < kCeWaves; ++w) {           // in wave order
+      s += sums[w];
+      n += counts[w];
+    }
+    *out = (float)(mean ? s / n : s);
+    *divisor = mean ? (float)n : 1.f;
   }
 }
 
