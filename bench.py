@@ -116,7 +116,7 @@ def gemm_bytes_per_token(d, P, cf, a=4, m=64, mc=64, fused=True):
 SURVEY_BYTES = {'cfg2': {'hip': 3340 + 4436, 'layer': 10680 + 15196},
                 'cfg3': {'hip': 2828 + 3860, 'layer': 24436}}
 # the library entry points whose kernels are K1-K5 (the clock scan runs forward and backward)
-K1_K5 = {'K1 hash + bucket sort': ['asrn_bucket_sort'], 'K2 clock': ['asrn_clock_scan'],
+K1_K5 = {'K1 hash + bucket sort': ['asrn_bucket_sort'], 'K2 clock': ['asrn_clock_scan', 'asrn_clock_bwd'],
          'K3 n-gram sort': ['asrn_ngram_sort'],
          'K4 Hawkes/streak scans': ['asrn_hawkes_fwd', 'asrn_hawkes_bwd', 'asrn_streak_fwd', 'asrn_streak_bwd',
                                     'asrn_repetition_fwd', 'asrn_repetition_bwd'],
@@ -357,20 +357,20 @@ def modelo_bench(dev, nombre, steps, warmup, seed=0, eager_steps=5):
             'skipped_last': float(salto)}
 
 
-def hip_aggregate(hip_b, tokens, eager_ms, prof_us):
-    """All HIP kernels' algorithmic bytes over their summed time per step: from the committed rocprofv3 kernel trace
+def hip_aggregate(hip_b, tokens, eager_ms, prof_us, config):
+    """All HIP kernels' algorithmic bytes (the dense products' left out) over their summed time per step: from the committed rocprofv3 kernel trace
     when there is one (the eager pass's event times include the host's launch gaps of a host-bound step), else from
     those events."""
     if prof_us:
         return {'bytes_per_token': hip_b, 'hip_us_per_step': prof_us, 'source': 'rocprofv3 kernel trace, '
-                'profiles/cfg2_kernel_times.json', 'frac': round(hip_b * tokens / (HBM_PEAK * prof_us * 1e-6), 4)}
+                f'profiles/{config}_kernel_times.json', 'frac': round(hip_b * tokens / (HBM_PEAK * prof_us * 1e-6), 4)}
     return {'bytes_per_token': hip_b, 'hip_us_per_step': round(eager_ms * 1e3, 1),
             'source': 'device events around each library call in the eager pass (include launch gaps)',
             'frac': round(hip_b * tokens / (HBM_PEAK * eager_ms * 1e-3), 4)}
 
 
 # kernel names (rocprofv3) of the K1-K5 groups and of the entry points whose traffic is reported
-K1_K5_KERNELS = {'K1 hash + bucket sort': ('k_bucket_',), 'K2 clock': ('ClockOp',),
+K1_K5_KERNELS = {'K1 hash + bucket sort': ('k_bucket_',), 'K2 clock': ('ClockOp', 'ClockBwd'),
                  'K3 n-gram sort': ('k_ngram_', 'k_merge_pass'),
                  'K4 Hawkes/streak scans': ('Hawkes', 'Streak', 'k_hawkes_'), 'K5 candidates': ('k_cand_',)}
 ENTRY_KERNELS = {'asrn_candidates_fwd': ('k_cand_fwd',), 'asrn_candidates_bwd': ('k_cand_bwd_q', 'k_cand_bwd_k'),
@@ -386,7 +386,8 @@ def _csv_rows(path):
 
 def summarize_trace(path, steps, command):
     """A rocprofv3 --kernel-trace --stats run (its directory) of `steps` traced steps -> the per-step summary that
-    profiles/<config>_kernel_times.json holds: all kernels, the HIP library's, and K1-K5 by group and kernel."""
+    profiles/<config>_kernel_times.json holds: all kernels, the HIP library's (its dense products, whose operands are
+    counted with the GEMMs', apart), and K1-K5 by group and kernel."""
     files, csv = _csv_rows(path)
     stats = [f for f in files if f.endswith('kernel_stats.csv')]
     if not stats:
@@ -400,7 +401,8 @@ def summarize_trace(path, steps, command):
         groups[g] = round(sum(ks.values()), 2)
         for n, us in ks.items():
             by_kernel[n.split('(')[0]] = {'us_per_step': round(us, 2), 'launches_per_step': calls[n]}
-    return {'hip_us_per_step': round(sum(us for n, us in per.items() if 'asrn::' in n), 1),
+    return {'hip_us_per_step': round(sum(us for n, us in per.items() if 'asrn::' in n and 'k_gemm' not in n), 1),
+            'products_us_per_step': round(sum(us for n, us in per.items() if 'asrn::k_gemm' in n), 1),
             'all_kernels_us_per_step': round(sum(per.values()), 1),
             'k1_k5_us_per_step': round(sum(groups.values()), 1), 'k1_k5_us_by_kernel': groups,
             'k1_k5_kernels': by_kernel, 'traced_steps': steps, 'source': command}
@@ -729,7 +731,7 @@ def main():
     dom = max(algo, key=lambda n: per_call.get(n, {}).get('total_ms', 0.0))
     dom_us = per_call[dom]['mean_us']
     achieved = algo[dom] * tokens / (dom_us * 1e-6)
-    hip_ms_per_step = sum(v['total_ms'] for v in per_call.values()) / args.steps
+    hip_ms_per_step = sum(v['total_ms'] for n, v in per_call.items() if n != 'asrn_gemm') / args.steps
     fused = not bf16                    # the fused hash kernels run in fp32 outside autocast
     hip_b = hip_bytes_per_token(d, P, cf, T, layer.vistos, a=2 if bf16 else 4, K=layer.sufijo, fused=fused)
     impl_b = hip_b + gemm_bytes_per_token(d, P, cf, a=2 if bf16 else 4, fused=fused)
@@ -748,7 +750,7 @@ def main():
                      'unit': 'GB/s', 'frac': round(achieved / HBM_PEAK, 4), 'traffic': measured_traffic(dom) if args.config == 'cfg2' else None,
                      'bytes_per_token': algo[dom], 'mean_launch_us': round(dom_us, 2)},
         'survey_headline': survey_headline(args.config, tokens, per_call, args.steps, kernel_times(args.config)),
-        'hip_aggregate': hip_aggregate(hip_b, tokens, hip_ms_per_step, profiled_hip_us(args.config)),
+        'hip_aggregate': hip_aggregate(hip_b, tokens, hip_ms_per_step, profiled_hip_us(args.config), args.config),
         'layer': {'tokens_per_s': round(value, 1),
                   'bytes_per_token': layer_b, 'hbm_frac': round(layer_b * tokens / (HBM_PEAK * wall), 4),
                   'bytes_source': "SURVEY.md 8(d)'s compulsory whole-layer bytes",
