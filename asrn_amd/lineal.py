@@ -179,7 +179,10 @@ class _Lineal(torch.autograd.Function):
     def forward(ctx, x, w, b, dt, propio):
         xc, wc = x.to(dt), w.to(dt)
         bc = b.to(dt) if b is not None else None
-        x2 = _rows(xc) if propio and xc.is_cuda and xc.dtype == torch.float32 else None
+        # rows flattened (which may copy) only for products that asrn_gemm takes by their size
+        x2 = None
+        if propio and xc.is_cuda and xc.dtype == torch.float32 and xc.numel() * wc.shape[0] >= MIN_PRODUCTO:
+            x2 = _rows(xc)
         if x2 is not None and gemm_ok(x2, wc, True, bc):
             y = gemm(x2, False, wc, True, sesgo=bc).view(*x.shape[:-1], wc.shape[0])
         else:
