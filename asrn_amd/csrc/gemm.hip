@@ -29,7 +29,7 @@
 // A workgroup of 4 waves forms a BM x BN tile, each wave a quarter of it from 32x32x16 MFMA tiles. Operands are loaded
 // into registers one step ahead, split there and stored to LDS in units of 8 consecutive k of one row, the operand an
 // MFMA lane takes; an operand stored with its rows contiguous (TA, TB) is transposed on the way, 8 k-rows per thread,
-// which costs nothing in fp32 and one permute per pair in bf16. Three workgroups share a CU in fp32 (49,920 bytes of LDS
+// which costs nothing in fp32 and one permute per pair in bf16. Three workgroups share a CU in fp32 (50,176 bytes of LDS
 // and 112 to 164 registers a wave): one's loads, splits and barriers run under the others' MFMA.
 // Products with few tiles (weight gradients: K is the token axis) are cut along K: partial products in a workspace,
 // summed in order by a second launch. No atomics: the result is a function of the sizes alone.
