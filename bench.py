@@ -87,13 +87,14 @@ def hip_bytes_per_token(d, P, cf, T, n=4, a=4, m=64, mc=64, K=4, fused=True):
     """All HIP kernels of one fwd+bwd, each distinct tensor read once and written once: sign hash + bucket sort (fused:
     the hash kernel writes the ids, the sort reads them and writes the order; else the sort reads phi and writes ids
     and order), clock 16 + 16, n-gram sort 28, Hawkes/streak scans 60 + 100, candidates, gate, context producer, the
-    hash MLPs (fused: hash_bytes; else the hidden layer and its bias column sums), and the column sums of the
+    hash MLPs (fused: hash_bytes; else the hidden layer and its bias column sums, and in 16 bits the key rows [E_t ; E_{t-1}]
+    and their gradients' sum: E in, rows and keys out, their three gradients in, dE out, 22 d), and the column sums of the
     candidates' per-token partials (the weight gradients' slab sums scale with the weights, not the tokens, and are
     left out).
     cfg2 fp32 (fused): 96 + 32 + 28 + 160 + 7,044 + 8,324 + 5,304 + 3,200 + 52 = 24,240."""
     cand = algorithmic_bytes(d, P, cf, T, a)
     colsums = 4 * (T + K + 1) + (0 if fused else 4 * (m + mc) + 4 * P)
-    mlp = sum(hash_bytes(P, m, mc)) if fused else sum(hidden_bytes(m, mc))
+    mlp = sum(hash_bytes(P, m, mc)) if fused else sum(hidden_bytes(m, mc)) + (22 * d if a == 2 else 0)
     return ((4 * T if fused else P * a) + 8 * T + 32 + 28 + 160 + sum(cand.values()) + sum(gate_bytes(d, n, a))
             + sum(context_bytes(d, cf, proj=fused)) + mlp + colsums)
 
